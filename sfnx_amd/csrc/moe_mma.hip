@@ -35,6 +35,15 @@ template <int SEL> __device__ __forceinline__ half2v bytes_1024(uint32_t w) {
     return as_h2(__builtin_amdgcn_perm(0x64646464u, w, SEL == 0 ? 0x05010400u : 0x05030402u));
 }
 
+// bytes 0, 1 (SEL 0) or 2, 3 (SEL 1) of w, each 0 .. 15, as two f16 values: as fp8 (e4m3) such a byte is the value times
+// 2^-9, exactly (0 .. 7 its subnormals, 8 .. 15 its first binade), and the conversion scales by 2^9.  One instruction, at
+// the full rate, where the byte permute and the subtraction of 1024 are two: a step's dequantization of 16 wavefronts
+// takes 330 ns for 460.  Q4_K gate|up + SwiGLU / down: 223 -> 198 / 131 -> 126 us at 2048 tokens (2048 columns, 512
+// experts), 121 -> 107 / 64 -> 58 us at 96.
+template <int SEL> __device__ __forceinline__ half2v nibbles_f16(uint32_t w) {
+    return __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, 512.0f, SEL != 0);
+}
+
 // Q4_K: 16 bytes of a group's quants (b0..b15, low nibbles of sub-block 2jg, high of 2jg + 1) -> the 4 B fragments;
 // Q5_K (qh given): the fifth bit of each value from bit j0 (low nibbles) or j0 + 1 (high) of the matching qh byte
 __device__ __forceinline__ void deq_q4k(const uint4& q, half2v d1l, half2v nml, half2v d1h, half2v nmh, half8 (&b)[4],
@@ -52,7 +61,8 @@ __device__ __forceinline__ void deq_q4k(const uint4& q, half2v d1l, half2v nml, 
         for (int p = 0; p < 2; ++p) {
             uint32_t v = hi ? (w[wi + p] >> 4) & 0x0F0F0F0Fu : w[wi + p] & 0x0F0F0F0Fu;
             if (qh) v |= ((x[wi + p] >> (hi ? j0 + 1 : j0)) & 0x01010101u) << 4;
-            const half2v q01 = bytes_1024<0>(v) - k1024, q23 = bytes_1024<1>(v) - k1024;
+            const half2v q01 = qh ? bytes_1024<0>(v) - k1024 : nibbles_f16<0>(v);
+            const half2v q23 = qh ? bytes_1024<1>(v) - k1024 : nibbles_f16<1>(v);
             const half2v r01 = __builtin_elementwise_fma(q01, d1, nm), r23 = __builtin_elementwise_fma(q23, d1, nm);
             b[c][4 * p + 0] = r01[0];
             b[c][4 * p + 1] = r01[1];
@@ -216,13 +226,14 @@ __device__ __forceinline__ void dequant_step(const Chunk<SFNX_Q5_K>& w, int s, h
     deq_q4k(w.q[s], half2v{D[0], D[0]}, half2v{N[0], N[0]}, half2v{D[1], D[1]}, half2v{N[1], N[1]}, b, &w.qh, 2 * s);
 }
 // Q4_0 / Q5_1: a block's 16 quant bytes (value l in the low nibble of byte l, l + 16 in the high) -> the 4 B
-// fragments, fragment c holding values 8 c .. 8 c + 7; Q4_0 hmul2(q - 8, d), Q5_1 hfma2(q, d, m) with the fifth bits
+// fragments, fragment c holding values 8 c .. 8 c + 7; Q4_0 hmul2(q - 8, d), as hfma2(q, d, -8 d) (-8 d is exact, so the one
+// rounding is of the same product), Q5_1 hfma2(q, d, m) with the fifth bits
 template <int TYPE>
 __device__ __forceinline__ void deq_nb(const uint4& q, uint32_t dm, uint32_t qh, half8 (&b)[4]) {
     const uint32_t w[4] = {q.x, q.y, q.z, q.w};
     const half2v d = {__builtin_bit_cast(_Float16, (uint16_t) (dm & 0xffff)), __builtin_bit_cast(_Float16, (uint16_t) (dm & 0xffff))};
-    const half2v m = {__builtin_bit_cast(_Float16, (uint16_t) (dm >> 16)), __builtin_bit_cast(_Float16, (uint16_t) (dm >> 16))};
-    const half2v off = TYPE == SFNX_Q4_0 ? half2v{(_Float16) 1032.0f, (_Float16) 1032.0f} : half2v{(_Float16) 1024.0f, (_Float16) 1024.0f};
+    const half2v k1024 = {(_Float16) 1024.0f, (_Float16) 1024.0f}, m8 = {(_Float16) -8.0f, (_Float16) -8.0f};
+    const half2v m = TYPE == SFNX_Q4_0 ? d * m8 : half2v{__builtin_bit_cast(_Float16, (uint16_t) (dm >> 16)), __builtin_bit_cast(_Float16, (uint16_t) (dm >> 16))};
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
         const bool hi = c >= 2;
@@ -231,15 +242,9 @@ __device__ __forceinline__ void deq_nb(const uint4& q, uint32_t dm, uint32_t qh,
             const int wi = 2 * (c % 2) + p;   // the dword: values 4 wi .. 4 wi + 3 (+ 16 for the high nibbles)
             uint32_t v = hi ? (w[wi] >> 4) & 0x0F0F0F0Fu : w[wi] & 0x0F0F0F0Fu;
             if constexpr (TYPE == SFNX_Q5_1) v |= spread4(qh >> ((hi ? 16 : 0) + 4 * wi));
-            const half2v q01 = bytes_1024<0>(v) - off, q23 = bytes_1024<1>(v) - off;
-            half2v r01, r23;
-            if constexpr (TYPE == SFNX_Q4_0) {
-                r01 = q01 * d;
-                r23 = q23 * d;
-            } else {
-                r01 = __builtin_elementwise_fma(q01, d, m);
-                r23 = __builtin_elementwise_fma(q23, d, m);
-            }
+            const half2v q01 = TYPE == SFNX_Q4_0 ? nibbles_f16<0>(v) : bytes_1024<0>(v) - k1024;
+            const half2v q23 = TYPE == SFNX_Q4_0 ? nibbles_f16<1>(v) : bytes_1024<1>(v) - k1024;
+            const half2v r01 = __builtin_elementwise_fma(q01, d, m), r23 = __builtin_elementwise_fma(q23, d, m);
             b[c][4 * p + 0] = r01[0];
             b[c][4 * p + 1] = r01[1];
             b[c][4 * p + 2] = r23[0];
