@@ -254,8 +254,10 @@ constexpr int RM_MIN_T = 512;
 constexpr int RM_WAVES = 8, RM_THREADS = RM_WAVES * WAVE, RM_RT = 3, RM_ROWS = 16 * RM_RT;
 constexpr int RM_PITCH = RM_ROWS + 1, RM_SLOTS = 2;
 typedef float float4v __attribute__((ext_vector_type(4)));
-// xh (may be null): x as f16 (round to nearest even) as well, written by the workgroups of the first row tile, whose
-// wavefronts between them read every value of their tokens' rows once
+// xh (may be null): x as f16 (round to nearest even) as well.  The row tiles of a token tile read the same values, so each
+// writes the steps that fall to it (step j: row tile j mod their number).  Written by the first row tile alone, its
+// workgroups ran 50 us where the others took 41, and the one-round launch with them (2048 tokens, 2048 columns, 513 rows:
+// 74 -> 64 us; 60 with the order of units below).
 template <int TOK>
 __global__ void __launch_bounds__(RM_THREADS) k_router_mm(const float* __restrict__ W, const float* __restrict__ x,
                                                          float* __restrict__ logits, int T, int H, int L,
@@ -264,7 +266,13 @@ __global__ void __launch_bounds__(RM_THREADS) k_router_mm(const float* __restric
     extern __shared__ __align__(16) unsigned char lds[];
     float* part = reinterpret_cast<float*>(lds);   // [RM_WAVES / 2][TOK][RM_PITCH]
     const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE, m = lane % 16, g = lane / 16;
-    const int r0 = blockIdx.x * RM_ROWS, t0 = blockIdx.y * TOK, KW = H / RM_WAVES, k0 = wave * KW + 4 * g;
+    // Workgroup b runs on XCD b % 8: each XCD takes one run of (token tile, row tile) units, the row tiles fastest, so that
+    // a token tile's activations are fetched into one or two XCDs' L2 and not into all eight (2048 tokens 64 -> 60 us, 4096
+    // 121 -> 115; a third operand slot in flight measured 81 and 140)
+    const int nrt = (L + RM_ROWS - 1) / RM_ROWS, units = nrt * ((T + TOK - 1) / TOK);
+    const int unit = (int) blockIdx.x % XCDS * ((units + XCDS - 1) / XCDS) + (int) blockIdx.x / XCDS;
+    if (unit >= units) return;
+    const int rt = unit % nrt, r0 = rt * RM_ROWS, t0 = unit / nrt * TOK, KW = H / RM_WAVES, k0 = wave * KW + 4 * g;
     const float4v* xa[TU];
     const float4v* wb[RM_RT];
 #pragma unroll
@@ -300,7 +308,7 @@ __global__ void __launch_bounds__(RM_THREADS) k_router_mm(const float* __restric
 #pragma unroll
                     for (int q = 0; q < RM_RT; ++q)
                         acc[u][q] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[sl][u][i], b[sl][q][i], acc[u][q], 0, 0, 0);
-            if (xh != nullptr && blockIdx.x == 0)
+            if (xh != nullptr && j % nrt == rt)
 #pragma unroll
                 for (int u = 0; u < TU; ++u)
                     if (t0 + 16 * u + m < T) {
@@ -716,7 +724,8 @@ void router_logits(const float* W, const float* x, float* logits, int T, int H, 
             const long nb = (long) rb * ((T + tk - 1) / tk), cost = (nb + ncu - 1) / ncu * round_us;
             if (tk == 32 || cost < best) tok = tk, best = cost;
         }
-        const dim3 g(rb, (T + tok - 1) / tok);
+        const int units = rb * ((T + tok - 1) / tok);
+        const dim3 g((units + XCDS - 1) / XCDS * XCDS);
         const size_t lds = (size_t) RM_WAVES / 2 * tok * RM_PITCH * 4;
         switch (tok) {
             case 32: k_router_mm<32><<<g, RM_THREADS, lds, st>>>(W, x, logits, T, H, L, xh); break;
