@@ -173,17 +173,25 @@ __global__ void __launch_bounds__(2 * d2_threads<TYPE>()) k_dec_experts(
     const sfnx_job* __restrict__ jg, const int* __restrict__ njobs_g, float* __restrict__ gu, int8_t* __restrict__ hq_q,
     float* __restrict__ hq_d, int* __restrict__ hq_s, Q8sPlanes sh_gu) {
     constexpr int LPR = lpr_of<TYPE>(), NTH = 2 * d2_threads<TYPE>(), NW = NTH / WAVE, RPW = WAVE / LPR;
-    const int NFB = ff / 32, fb = blockIdx.x % NFB, nj = njobs_g[0];
+    const int NFB = ff / 32, fb = blockIdx.x % NFB, unit = blockIdx.x / NFB;
     const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
     __shared__ sfnx_job jb;
     __shared__ float gbuf[SFNX_MAXT][32], ubuf[SFNX_MAXT][32];
     extern __shared__ __align__(16) unsigned char lds[];
-    if ((int) blockIdx.x / NFB >= nj) return;
     // the last job first: with a shared expert it is the shared job, which holds every row of the window and so takes
-    // the longest (2.5x a routed job's blocks at 16 rows); dispatched last, its blocks ran alone at the kernel's end
-    const int myjob = ((int) blockIdx.x / NFB + nj - 1) % nj;
-    load_job(jb, jg + myjob);
-    __syncthreads();
+    // the longest (2.5x a routed job's blocks at 16 rows); dispatched last, its blocks ran alone at the kernel's end.
+    // The other units' job does not depend on the job count, so its words, its expert and the count are requested together
+    static_assert(sizeof(sfnx_job) / 4 <= WAVE, "a wavefront loads a job");
+    int nj = njobs_g[0], ex = jg[unit ? unit - 1 : 0].w;
+    int word = reinterpret_cast<const int*>(jg + (unit ? unit - 1 : 0))[min(lane, (int) (sizeof(sfnx_job) / 4) - 1)];
+    asm volatile("" : "+s"(nj), "+s"(ex));
+    if (unit >= nj) return;
+    if (unit == 0) {
+        ex = jg[nj - 1].w;
+        word = reinterpret_cast<const int*>(jg + nj - 1)[min(lane, (int) (sizeof(sfnx_job) / 4) - 1)];
+    }
+    if (threadIdx.x < sizeof(sfnx_job) / 4) reinterpret_cast<int*>(&jb)[threadIdx.x] = word;
+    lds_barrier();
     const bool up = wave >= NW / 2;
     const int rw = lane / LPR, ln = lane % LPR, fl = (up ? wave - NW / 2 : wave) * RPW + rw, row = (up ? ff : 0) + fb * 32 + fl;
     auto put = [&](int s, float v) {
@@ -194,12 +202,13 @@ __global__ void __launch_bounds__(2 * d2_threads<TYPE>()) k_dec_experts(
     };
     // the weight rows are requested first, then the job's rows of activations staged (slot s holds row jb.y[s]): the
     // two fetches overlap instead of following each other
-    const bool dense_sh = sh_gu.q != nullptr && jb.w == E;   // the shared expert's own dense Q8_0 matrix
+    const bool dense_sh = sh_gu.q != nullptr && ex == E;   // the shared expert's own dense Q8_0 matrix
     typename RowOf<TYPE, G>::R w;
-    if (!dense_sh) RowOf<TYPE, G>::load(w, expert_at(A, sa, jb.w), 2 * ff, row, H, ln);
+    if (!dense_sh) RowOf<TYPE, G>::issue(w, expert_at(A, sa, ex), 2 * ff, row, H, ln);
     const Acts a = acts_in(lds, TT, H);
     stage_q8_1(a, xq, jb.y, jb.n);
-    __syncthreads();   // the staged activations
+    lds_barrier();   // the staged activations
+    if (!dense_sh) w.prepare(ln);
     if (dense_sh) {   // the reference's q8s sums
         const Q8sPlanes Ps = sh_gu;
         for (int s = 0; s < jb.n; ++s) put(s, group_sum<LPR>(q8s_dot<LPR>(Ps, row, H, ln, a, s)));
@@ -350,27 +359,35 @@ __global__ void __launch_bounds__(2 * d2_threads<TYPE>()) k_dec_experts1(
 }
 
 // ------------------------------------------------------------------------------------------------ K3
-// (windows: 512 threads, twice the lane groups of the batch-1 kernel, so a group takes half the tasks)
-template <int TYPE, int G2, int NB, int NT>
-__global__ void __launch_bounds__(NT) k_dec_down(const uint8_t* __restrict__ A, size_t sa, int T, int H, int E, int K,
+// LDS of a window's jobs (whole 16-byte pieces: the job array's piece of the workspace is a multiple of 256 bytes)
+__host__ __device__ constexpr size_t d3_jobs_bytes(int njmax) { return (njmax * sizeof(sfnx_job) + 15) / 16 * 16; }
+// Windows: 512 or 1024 threads; the wavefronts take (job, rows) units from a queue.  Bound by the down rows' bytes and by the
+// chain of dots of the wavefront that finishes last: with the tasks dealt out in turn the first wavefront ended the 16-row
+// window's dots at 14.6 us and the last, which held the shared expert's 16 pairs beside its share, at 21.9.  Measured, 16
+// rows (2048 columns, 512 experts, Q4_K) 27.4 -> 24.2 us; 5 rows (2560 columns, FF 1024, Q8_0 down, 128 registers
+// instead of 155, so that two workgroups share a compute unit) 38.0 -> 26.5 us.
+template <int TYPE, int G2, int NT>
+__global__ void __launch_bounds__(NT, NT == 512 && is_kquant(TYPE) ? 2 : 4) k_dec_down(const uint8_t* __restrict__ A, size_t sa, int T, int H, int E, int K,
                                                         int ff, int shared, const float* __restrict__ logits,
                                                         const int* __restrict__ topi, const float* __restrict__ topw,
                                                         const sfnx_job* __restrict__ jd, const int* __restrict__ njobs,
                                                         const int8_t* __restrict__ hq_q, const float* __restrict__ hq_d,
                                                         const int* __restrict__ hq_s, float* __restrict__ y,
                                                         float* __restrict__ x, int hq_in_lds, Q8sPlanes sh_dn) {
-    constexpr int LPR = lpr_of<TYPE>(), GROUPS = NT / LPR;
-    const int row0 = blockIdx.x * D3_ROWS, nj = njobs[0], P = T * K, NP = P + T, nbh = ff / 32;
-    __shared__ int jw[MAX_P + 1], jn[MAX_P + 1], jout[MAX_P + 1][SFNX_MAXT];
+    constexpr int LPR = lpr_of<TYPE>(), GROUPS = NT / LPR, NWV = NT / WAVE, RING = G2 == 1 ? 3 : 2;
+    const int row0 = blockIdx.x * D3_ROWS, P = T * K, NP = P + T, nbh = ff / 32, njmax = P + (shared ? 1 : 0);
     __shared__ float part[MAX_P + SFNX_MAXT][D3_ROWS];
     __shared__ int ti[MAX_P];
     __shared__ float tw[MAX_P], sg[SFNX_MAXT];
-    extern __shared__ __align__(16) unsigned char lds[];   // every pair's h, when the launch gave room for it
-    for (int i = threadIdx.x; i < nj; i += NT) {
-        jw[i] = jd[i].w;
-        jn[i] = jd[i].n;
-        for (int s = 0; s < jd[i].n; ++s) jout[i][s] = jd[i].out[s];
-    }
+    __shared__ int queue;
+    extern __shared__ __align__(16) unsigned char lds[];   // the window's jobs, then every pair's h when the launch gave room
+    const int wv = threadIdx.x / WAVE, ln64 = threadIdx.x % WAVE;
+    // the jobs as they are (no more than the window can have, so nothing waits for their count), by asynchronous copies
+    const sfnx_job* jobs = reinterpret_cast<const sfnx_job*>(lds);
+    const int jw16 = (int) d3_jobs_bytes(njmax) / 16;
+    for (int c = wv; c * WAVE < jw16; c += NWV)
+        if (c * WAVE + ln64 < jw16) lds_copy_async<16>(reinterpret_cast<const uint4*>(jd) + c * WAVE + ln64, lds + 16 * (size_t) c * WAVE);
+    const int nj = njobs[0];
     for (int i = threadIdx.x; i < P; i += NT) {
         ti[i] = topi[i];
         tw[i] = topw[i];
@@ -379,30 +396,47 @@ __global__ void __launch_bounds__(NT) k_dec_down(const uint8_t* __restrict__ A, 
     for (int i = threadIdx.x; i < T * D3_ROWS; i += NT) xr[i / D3_ROWS][i % D3_ROWS] = x[(size_t) (i / D3_ROWS) * H + row0 + i % D3_ROWS];
     if (shared)
         for (int t = threadIdx.x; t < T; t += NT) sg[t] = sigm_f(logits[(size_t) t * (E + 1) + E]);
-    Acts a;
+    vm_wait<0>();
+    lds_barrier();
     const bool staged = hq_in_lds != 0;
-    if (staged) {
-        // every pair's h into LDS by asynchronous global -> LDS copies, all issued before one wait (a copy loop through
-        // registers would wait for each of its ~11 rounds in turn): wavefront w copies chunks of 64 lanes, 16 bytes
-        // (values) or 4 bytes (scales, sums) a lane
-        a = acts_in(lds, NP, ff);
-        const int wv = threadIdx.x / WAVE, ln64 = threadIdx.x % WAVE;
-        constexpr int NWV = NT / WAVE;
-        for (int c = wv; c * WAVE < NP * ff / 16; c += NWV)
-            if (c * WAVE + ln64 < NP * ff / 16)
-                __builtin_amdgcn_global_load_lds(hq_q + 16 * ((size_t) c * WAVE + ln64),
-                                                 (__attribute__((address_space(3))) void*) (a.q + 16 * (size_t) c * WAVE), 16, 0, 0);
-        for (int c = wv; c * WAVE < NP * nbh; c += NWV)
-            if (c * WAVE + ln64 < NP * nbh) {
-                __builtin_amdgcn_global_load_lds(hq_d + c * WAVE + ln64, (__attribute__((address_space(3))) void*) (a.d + c * WAVE), 4, 0, 0);
-                __builtin_amdgcn_global_load_lds(hq_s + c * WAVE + ln64, (__attribute__((address_space(3))) void*) (a.s + c * WAVE), 4, 0, 0);
-            }
-        __builtin_amdgcn_s_waitcnt(0);   // the copies landed (vmcnt), before the barrier below
-    }
-    __syncthreads();
     const int g = threadIdx.x / LPR, ln = threadIdx.x % LPR;
     // with its own dense Q8_0 matrix the shared expert's job (the last) runs apart, in the reference's q8s sums
     const int nq = sh_dn.q != nullptr && shared ? nj - 1 : nj, ntask = nq * D3_ROWS;
+    // every pair's h into LDS by asynchronous global -> LDS copies: wavefront w copies chunks of 64 lanes, 16 bytes
+    // (values) or 4 bytes (scales, sums) a lane
+    const Acts a = acts_in(lds + d3_jobs_bytes(njmax), NP, ff);
+    if (staged) {
+        for (int c = wv; c * WAVE < NP * ff / 16; c += NWV)
+            if (c * WAVE + ln64 < NP * ff / 16) lds_copy_async<16>(hq_q + 16 * ((size_t) c * WAVE + ln64), a.q + 16 * (size_t) c * WAVE);
+        for (int c = wv; c * WAVE < NP * nbh; c += NWV)
+            if (c * WAVE + ln64 < NP * nbh) {
+                lds_copy_async<4>(hq_d + c * WAVE + ln64, a.d + c * WAVE);
+                lds_copy_async<4>(hq_s + c * WAVE + ln64, a.s + c * WAVE);
+            }
+    }
+    // A unit: a wavefront's rows of one job (a lane group a row).  Each wavefront takes two units, then the next of the
+    // block's queue as it finishes one, so the window's longest job (the shared expert's, first here) does not leave its
+    // wavefront behind.  A unit's weight rows are requested RING - 1 units before they are dotted, the first ones with h
+    // (its wait below covers both); units past the last request its rows again, so that each turn's requests are the same
+    constexpr int UPJ = D3_ROWS * LPR / WAVE;   // units a job
+    static_assert(UPJ >= 1, "a wavefront holds at most a job's rows");
+    const int nunit = nq * UPJ, gw = ln64 / LPR;
+    typename RowOf<TYPE, G2>::R w[RING];
+    int u[RING];
+    auto row_of = [&](int unit) { return unit % UPJ * (WAVE / LPR) + gw; };
+    auto job_of = [&](int unit) -> const sfnx_job& { return jobs[nq - 1 - unit / UPJ]; };
+    auto request = [&](typename RowOf<TYPE, G2>::R& v, int unit) {
+        const int c = min(unit, nunit - 1), e = __builtin_amdgcn_readfirstlane(job_of(c).w);
+        RowOf<TYPE, G2>::issue(v, expert_at(A, sa, e), H, row0 + row_of(c), ff, ln);
+    };
+    if (threadIdx.x == 0) queue = (RING - 1) * NWV;
+#pragma unroll
+    for (int k = 0; k < RING - 1; ++k) {
+        u[k] = wv + k * NWV;
+        if (nunit > 0) request(w[k], u[k]);
+    }
+    vm_wait<0>();
+    lds_barrier();
     // the dots, inlined once for h in LDS and once for h in global memory: a pointer that may be either is generic,
     // and every load through it a flat load
     auto dots = [&](const Acts& a) __attribute__((always_inline)) {
@@ -414,26 +448,25 @@ __global__ void __launch_bounds__(NT) k_dec_down(const uint8_t* __restrict__ A, 
             if (ln == 0) part[P + t][r] = v;
         }
     }
-    for (int t0 = g; t0 < ntask; t0 += GROUPS * NB) {
-        typename RowOf<TYPE, G2>::R w[NB];
+    for (bool more = true; more;) {
 #pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            const int task = t0 + b * GROUPS;
-            if (task < ntask) {
-                const int j = task / D3_ROWS, r = task % D3_ROWS;
-                RowOf<TYPE, G2>::load(w[b], expert_at(A, sa, jw[j]), H, row0 + r, ff, ln);
+        for (int k = 0; k < RING; ++k) {
+            if (u[k] >= nunit) {   // a wavefront's units only grow: the ones after are past the last too
+                more = false;
+                break;
             }
-        }
-#pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            const int task = t0 + b * GROUPS;
-            if (task < ntask) {
-                const int j = task / D3_ROWS, r = task % D3_ROWS;
-                for (int s = 0; s < jn[j]; ++s) {
-                    const int pp = jout[j][s];
-                    const float v = group_sum<LPR>(w[b].dot(a, pp, ln));
-                    if (ln == 0) part[pp][r] = v;
-                }
+            constexpr int AHEAD = RING - 1;
+            int nx = 0;
+            if (ln64 == 0) nx = atomicAdd(&queue, 1);
+            u[(k + AHEAD) % RING] = __builtin_amdgcn_readfirstlane(nx);
+            request(w[(k + AHEAD) % RING], u[(k + AHEAD) % RING]);
+            w[k].prepare(ln);
+            const sfnx_job& j = job_of(u[k]);
+            const int n = __builtin_amdgcn_readfirstlane(j.n), r = row_of(u[k]);
+            for (int s = 0; s < n; ++s) {
+                const int pp = j.out[s];
+                const float v = group_sum<LPR>(w[k].dot(a, pp, ln));
+                if (ln == 0) part[pp][r] = v;
             }
         }
     }
@@ -659,24 +692,24 @@ void launch_k3_one(const DecArgs& d, const sfnx_moe_layer_w& w, float* x, const 
         (const float*) (ws + L.hq_d), (const int*) (ws + L.hq_s), (float*) (ws + L.y), x, (const int*) (ws + L.route_x),
         d.sh_dn);
 }
-template <int TYPE, int G2, int NB>
+template <int TYPE, int G2>
 void launch_k3(const DecArgs& d, const sfnx_moe_layer_w& w, float* x, const DecLayout& L, char* ws, hipStream_t s) {
     if (d.T == 1) {
         launch_k3_one<TYPE, G2>(d, w, x, L, ws, s);
         return;
     }
     const int NP = d.T * d.K + d.T;
-    const size_t hq_lds = acts_bytes(NP, d.ff);
-    // every pair's h in LDS when it fits beside the kernel's own ~30 KB (160 KB a workgroup on gfx950; past 64 KB the
-    // kernel must be allowed the larger dynamic size first), else read from L2 per task
-    constexpr size_t HQ_LDS_MAX = 120 * 1024;
+    const size_t job_lds = d3_jobs_bytes(d.T * d.K + (d.shared ? 1 : 0)), hq_lds = job_lds + acts_bytes(NP, d.ff);
+    // every pair's h in LDS when it fits beside the jobs and the kernel's own ~12 KB (160 KB a workgroup on gfx950; past
+    // 64 KB the kernel must be allowed the larger dynamic size first), else read from L2 per task
+    constexpr size_t DYN_MAX = 144 * 1024;
     // 1024 threads (4 wavefronts a SIMD: the per-pair dot chains are latency-bound) where 128 registers hold a lane's
     // tasks (FF 512; not Q5_K, whose rows carry their fifth bits)
     constexpr int NT = G2 == 1 && TYPE != SFNX_Q5_K ? 1024 : 512;
-    static bool big_lds = hipFuncSetAttribute((const void*) k_dec_down<TYPE, G2, NB, NT>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                              (int) HQ_LDS_MAX) == hipSuccess;
-    const bool staged = hq_lds <= (big_lds ? HQ_LDS_MAX : 32 * 1024);
-    launch(2, k_dec_down<TYPE, G2, NB, NT>, dim3(d.H / D3_ROWS), dim3(NT), staged ? hq_lds : 0, s,
+    static bool big_lds = hipFuncSetAttribute((const void*) k_dec_down<TYPE, G2, NT>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                              (int) DYN_MAX) == hipSuccess;
+    const bool staged = hq_lds <= (big_lds ? DYN_MAX : 32 * 1024);
+    launch(2, k_dec_down<TYPE, G2, NT>, dim3(d.H / D3_ROWS), dim3(NT), staged ? hq_lds : job_lds, s,
         (const uint8_t*) w.dn, w.dn_stride, d.T, d.H, d.E, d.K, d.ff, d.shared, (const float*) (ws + L.logits),
         (const int*) (ws + L.topi), (const float*) (ws + L.topw), (const sfnx_job*) (ws + L.jd), (const int*) (ws + L.njobs),
         (const int8_t*) (ws + L.hq_q), (const float*) (ws + L.hq_d), (const int*) (ws + L.hq_s), (float*) (ws + L.y), x,
@@ -711,24 +744,22 @@ void launch_layer_tt(const DecArgs& d, const sfnx_moe_layer_w& w, float* x, cons
         }
     }
 #undef SFNX_K2
-    // down tasks a lane group loads together: every job's 8 rows in one batch at T = 1
-    constexpr int NB = TT == 1 ? 3 : 4, NB2 = NB;
     if (!(d.phases & 4)) return;
     if (d.dn_type == SFNX_Q4_K) {
-        if (d.ff == 512) launch_k3<SFNX_Q4_K, 1, NB>(d, w, x, L, ws, s);
-        else launch_k3<SFNX_Q4_K, 2, NB2>(d, w, x, L, ws, s);
+        if (d.ff == 512) launch_k3<SFNX_Q4_K, 1>(d, w, x, L, ws, s);
+        else launch_k3<SFNX_Q4_K, 2>(d, w, x, L, ws, s);
     } else if (d.dn_type == SFNX_Q5_K) {
-        if (d.ff == 512) launch_k3<SFNX_Q5_K, 1, NB>(d, w, x, L, ws, s);
-        else launch_k3<SFNX_Q5_K, 2, NB2>(d, w, x, L, ws, s);
+        if (d.ff == 512) launch_k3<SFNX_Q5_K, 1>(d, w, x, L, ws, s);
+        else launch_k3<SFNX_Q5_K, 2>(d, w, x, L, ws, s);
     } else if (d.dn_type == SFNX_Q4_0) {
-        if (d.ff == 512) launch_k3<SFNX_Q4_0, 1, NB>(d, w, x, L, ws, s);
-        else launch_k3<SFNX_Q4_0, 2, NB2>(d, w, x, L, ws, s);
+        if (d.ff == 512) launch_k3<SFNX_Q4_0, 1>(d, w, x, L, ws, s);
+        else launch_k3<SFNX_Q4_0, 2>(d, w, x, L, ws, s);
     } else if (d.dn_type == SFNX_Q5_1) {
-        if (d.ff == 512) launch_k3<SFNX_Q5_1, 1, NB>(d, w, x, L, ws, s);
-        else launch_k3<SFNX_Q5_1, 2, NB2>(d, w, x, L, ws, s);
+        if (d.ff == 512) launch_k3<SFNX_Q5_1, 1>(d, w, x, L, ws, s);
+        else launch_k3<SFNX_Q5_1, 2>(d, w, x, L, ws, s);
     } else {
-        if (d.ff == 512) launch_k3<SFNX_Q8_0, 1, NB>(d, w, x, L, ws, s);
-        else launch_k3<SFNX_Q8_0, 2, NB2>(d, w, x, L, ws, s);
+        if (d.ff == 512) launch_k3<SFNX_Q8_0, 1>(d, w, x, L, ws, s);
+        else launch_k3<SFNX_Q8_0, 2>(d, w, x, L, ws, s);
     }
 }
 
