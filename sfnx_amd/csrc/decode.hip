@@ -213,7 +213,13 @@ __global__ void __launch_bounds__(2 * d2_threads<TYPE>()) k_dec_experts(
         const Q8sPlanes Ps = sh_gu;
         for (int s = 0; s < jb.n; ++s) put(s, group_sum<LPR>(q8s_dot<LPR>(Ps, row, H, ln, a, s)));
     } else {
-        for (int s = 0; s < jb.n; ++s) put(s, group_sum<LPR>(w.dot(a, s, ln)));
+        // (most jobs hold one or two rows: the nibbles split anew for each cost less than the registers of a split row.
+        // Q4_K at 2048 columns 128 -> 75 registers, three workgroups a compute unit: 38.8 -> 34.9 us at 16 rows; Q5_K at
+        // 2560 columns 150 -> 126, two: 42.0 -> 34.5 us at 5 rows)
+        for (int s = 0; s < jb.n; ++s) {
+            if constexpr (is_kquant(TYPE)) w.pin();
+            put(s, group_sum<LPR>(w.dot(a, s, ln)));
+        }
     }
     __syncthreads();
     for (int s = threadIdx.x / 32; s < jb.n; s += NTH / 32) {

@@ -81,7 +81,9 @@ template <int GPL, bool Q5 = false> struct Q4kRow {
     uint4 q0[GPL], q1[GPL];
     uint4 h[GPL];
     uint4 qh0[Q5 ? GPL : 1], qh1[Q5 ? GPL : 1];
-    float d[GPL], dmin[GPL], sc0[GPL], m0[GPL], sc1[GPL], m1[GPL];
+    // a prepared header: this lane's two sub-blocks' 6-bit scales and mins as bytes (sc0, m0, sc1, m1) beside h.x (f16 d,
+    // dmin), 2 registers a group where six floats would make the wide rows' kernels hold one workgroup a compute unit
+    uint32_t scm[GPL];
     // the loads alone (issue several rows' before any prepare, so that their latencies overlap)
     // P: the planar store's planes (Q4kPlanes), or any view with the same accessors (one row staged in LDS)
     template <typename PL> __device__ __forceinline__ void issue(const PL& P, int row, int C, int l8) {
@@ -96,19 +98,33 @@ template <int GPL, bool Q5 = false> struct Q4kRow {
             }
         }
     }
-    // the block headers decoded: d, dmin and this lane's two sub-blocks' 6-bit scales and mins
+    // group i's header decoded (q4k_scale_min of sub-blocks 2 (l8 & 3) and the next)
+    __device__ __forceinline__ void prepare1(int i, int l8) {
+        const int j = 2 * (l8 & 3), sh = 8 * (j & 3);
+        const uint32_t y = h[i].y >> sh, z = h[i].z >> sh, w = h[i].w >> sh;   // bytes of sub-blocks j and j + 1 (mod 4)
+        const uint32_t sc = j < 4 ? y & 0x3F3Fu : (w & 0x0F0Fu) | ((y >> 2) & 0x3030u);
+        const uint32_t m = j < 4 ? z & 0x3F3Fu : ((w >> 4) & 0x0F0Fu) | ((z >> 2) & 0x3030u);
+        scm[i] = __builtin_amdgcn_perm(m, sc, 0x05010400u);
+    }
     __device__ __forceinline__ void prepare(int l8) {
 #pragma unroll
-        for (int i = 0; i < GPL; ++i) {
-            d[i] = h2f((uint16_t) (h[i].x & 0xffff));
-            dmin[i] = h2f((uint16_t) (h[i].x >> 16));
-            q4k_scale_min(h[i], 2 * (l8 & 3), sc0[i], m0[i]);
-            q4k_scale_min(h[i], 2 * (l8 & 3) + 1, sc1[i], m1[i]);
-        }
+        for (int i = 0; i < GPL; ++i) prepare1(i, l8);
     }
     __device__ __forceinline__ void load(const Q4kPlanes& P, int row, int C, int l8) {
         issue(P, row, C, l8);
         prepare(l8);
+    }
+    // keeps the compiler from splitting the nibbles and scales once before a loop of dots, which takes three times their
+    // registers
+    __device__ __forceinline__ void pin() {
+#pragma unroll
+        for (int i = 0; i < GPL; ++i) {
+            asm volatile("" : "+v"(q0[i].x), "+v"(q0[i].y), "+v"(q0[i].z), "+v"(q0[i].w), "+v"(q1[i].x), "+v"(q1[i].y),
+                              "+v"(q1[i].z), "+v"(q1[i].w), "+v"(h[i].x), "+v"(scm[i]));
+            if constexpr (Q5)
+                asm volatile("" : "+v"(qh0[i].x), "+v"(qh0[i].y), "+v"(qh0[i].z), "+v"(qh0[i].w), "+v"(qh1[i].x),
+                                  "+v"(qh1[i].y), "+v"(qh1[i].z), "+v"(qh1[i].w));
+        }
     }
     // prepare() and dot(a, 0, l8) in one pass: a group's header decoded as the group is reached, so the work on the
     // first groups overlaps the arrival of the later ones (the same values as prepare() then dot())
@@ -116,10 +132,7 @@ template <int GPL, bool Q5 = false> struct Q4kRow {
         float tmp = 0.f;
 #pragma unroll
         for (int i = 0; i < GPL; ++i) {
-            d[i] = h2f((uint16_t) (h[i].x & 0xffff));
-            dmin[i] = h2f((uint16_t) (h[i].x >> 16));
-            q4k_scale_min(h[i], 2 * (l8 & 3), sc0[i], m0[i]);
-            q4k_scale_min(h[i], 2 * (l8 & 3) + 1, sc1[i], m1[i]);
+            prepare1(i, l8);
             tmp += group(a, 0, l8, i);
         }
         return tmp;
@@ -147,8 +160,10 @@ template <int GPL, bool Q5 = false> struct Q4kRow {
         const int nb = a.K / 32;
         const float d8l = a.d[j * nb + kb0], d8h = a.d[j * nb + kb0 + 1];
         const float sl = (float) a.s[j * nb + kb0], sh = (float) a.s[j * nb + kb0 + 1];
-        return d[i] * (d8l * (sc0[i] * (float) dl) + d8h * (sc1[i] * (float) dh)) -
-               dmin[i] * (d8l * (m0[i] * sl) + d8h * (m1[i] * sh));
+        const float d = h2f((uint16_t) (h[i].x & 0xffff)), dmin = h2f((uint16_t) (h[i].x >> 16));
+        const float sc0 = (float) (scm[i] & 0xff), m0 = (float) ((scm[i] >> 8) & 0xff);
+        const float sc1 = (float) ((scm[i] >> 16) & 0xff), m1 = (float) (scm[i] >> 24);
+        return d * (d8l * (sc0 * (float) dl) + d8h * (sc1 * (float) dh)) - dmin * (d8l * (m0 * sl) + d8h * (m1 * sh));
     }
     // this lane's share of row . activation row j
     __device__ __forceinline__ float dot(const Acts& a, int j, int l8) const {
