@@ -60,7 +60,10 @@ __device__ __forceinline__ void deq_q4k(const uint4& q, half2v d1l, half2v nml, 
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
             uint32_t v = hi ? (w[wi + p] >> 4) & 0x0F0F0F0Fu : w[wi + p] & 0x0F0F0F0Fu;
-            if (qh) v |= ((x[wi + p] >> (hi ? j0 + 1 : j0)) & 0x01010101u) << 4;
+            if (qh) {   // bit j of each qh byte to bit 4 (one mask, folded into the OR)
+                const int j = hi ? j0 + 1 : j0;
+                v |= (j < 4 ? x[wi + p] << (4 - j) : x[wi + p] >> (j - 4)) & 0x10101010u;
+            }
             const half2v q01 = qh ? bytes_1024<0>(v) - k1024 : nibbles_f16<0>(v);
             const half2v q23 = qh ? bytes_1024<1>(v) - k1024 : nibbles_f16<1>(v);
             const half2v r01 = __builtin_elementwise_fma(q01, d1, nm), r23 = __builtin_elementwise_fma(q23, d1, nm);

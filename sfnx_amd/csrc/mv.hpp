@@ -227,8 +227,10 @@ template <int BPL> struct Q80Row {
 
 // ------------------------------------------------------------------------------------------------ Q4_0, Q5_1
 // bits 0..3 of t to bit 4 of bytes 0..3
+// (a 24-bit product puts a copy of the 4 bits every 7 bits, so bit k of the copy at 7 k is bit 8 k of the product: 4
+// instructions for 11.  Q5_1 prompt gate|up / down, 2048 tokens: 315 -> 245 / 168 -> 151 us)
 __device__ __forceinline__ uint32_t spread4(uint32_t t) {
-    return ((t & 1u) << 4) | ((t & 2u) << 11) | ((t & 4u) << 18) | ((t & 8u) << 25);
+    return (__umul24(t & 0xFu, 0x204081u) & 0x01010101u) << 4;
 }
 // The Q8_0 lanes (16 a row, lane l16 the blocks l16 + 16 i in order).  Per block the exact integer dot of the values
 // (Q5_1: the fifth bit of value l is qh bit l) with the activation block, then Q4_0 (d_w d_a) (sum - 8 s), Q5_1
