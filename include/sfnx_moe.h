@@ -93,7 +93,7 @@ int sfnx_quantize_q8_1(const float* x, void* q, int n, int rows, void* st);
  * gates the shared expert); top-K per token among the first E by logit, ties to the lower index; weights the selected
  * softmax renormalised; jobs: one per distinct expert in first-pick order, rows in pair order (pair p = t K + k:
  * gu.y = t, gu.out = dn.y = dn.out = p).  shared != 0: one more job, expert E, rows t -> T K + t.  njobs[0] = job
- * count; njobs[1] is the launch's block counter and must be 0 before the first call (every call leaves it 0).
+ * count; njobs[1] = 0.
  * H % 256 == 0, H <= 4096; E % 64 == 0, E <= 1024; 1 <= K <= 16.  Pick rounds with nothing left (NaN / -inf logits)
  * write topi -1, topw 0 and leave the pair out of the jobs. */
 int sfnx_router_route(const float* W, const float* x, float* logits, int T, int H, int E, int K, int* topi, float* topw,
@@ -365,8 +365,8 @@ int sfnx_host_free(void* host);
  * their slots, and status[0] receives the count (the reference's plan would spin).  Every slot the window holds ends
  * at ref 1 either way. */
 int sfnx_cache_plan(const sfnx_job* jobs, const int* njobs, int layer, const sfnx_expert_cache* ec, int* list, void* st);
-/* src/kernels.hpp:269-278 router_route with an ExpertCache (src/moe.cuh:128-198): sfnx_router_route, and then, in
- * the same launch, its last block's first wavefront plans the window's slots for `layer` as sfnx_cache_plan does (the
+/* src/kernels.hpp:269-278 router_route with an ExpertCache (src/moe.cuh:128-198): sfnx_router_route, whose
+ * routing launch's first wavefront then plans the window's slots for `layer` as sfnx_cache_plan does (the
  * same slots, list, tables, refs, hand and status), so a cached layer's plan takes no launch of its own.  With shared
  * != 0 the shared job (expert E) is planned like the others, so the cache's tables need E + 1 experts a layer. */
 int sfnx_router_route_plan(const float* W, const float* x, float* logits, int T, int H, int E, int K, int* topi,

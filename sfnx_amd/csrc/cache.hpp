@@ -1,5 +1,5 @@
 // The expert cache's window plan (src/moe.cuh:22-71 cache_plan) as a device function of one wavefront, run by the
-// plan kernel of its own (cache.hip) and by the last block of the decode router (route.hip), as the reference runs it.
+// plan kernel of its own (cache.hip) and by the decode routing's one workgroup (route.hip), as the reference runs it.
 #pragma once
 #include "common.hpp"
 

@@ -138,11 +138,6 @@ __device__ __forceinline__ void q4k_scale_min(const uint4& h, int j, float& sc, 
     }
 }
 
-// agent-scope loads for data another workgroup wrote earlier in the same launch
-__device__ __forceinline__ float load_agent(const float* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 // ------------------------------------------------------------------------------------------------ async LDS copies
 // Global -> LDS copies (global_load_lds) issued as inline assembly, so the compiler does not track them: it tracks such
 // copies per wavefront, not per LDS object, and with one in flight it makes the next LDS read wait for every vector

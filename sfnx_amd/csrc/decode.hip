@@ -16,6 +16,7 @@
 #include <mutex>
 
 #include "decode.hpp"
+#include "route_jobs.hpp"
 
 namespace sfnx {
 namespace {
@@ -109,61 +110,6 @@ __global__ void __launch_bounds__(D1_THREADS * d1_groups<TT>()) k_dec_router(con
 }
 
 // ------------------------------------------------------------------------------------------------ K2
-// K1b for windows of several rows: the routing once (the top-k of every row, a wavefront a row, then the decode job
-// numbering of src/moe.cuh:164-198), published for K2, K3 and the caller.  At batch 1, K2's blocks take the top-k
-// themselves (k_dec_experts1); with more rows each block would repeat every row's top-k and the numbering.
-constexpr int DR_THREADS = 1024;   // a wavefront per row (T <= 16) and a thread per pick
-__global__ void __launch_bounds__(DR_THREADS) k_dec_route(int T, int E, int K, int shared, const float* __restrict__ logits,
-                                                          int* __restrict__ topi_g, float* __restrict__ topw_g,
-                                                          sfnx_job* __restrict__ jg, sfnx_job* __restrict__ jd,
-                                                          int* __restrict__ njobs_g) {
-    constexpr int NW = DR_THREADS / WAVE;
-    const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE, p = threadIdx.x, P = T * K;
-    __shared__ int ex[MAX_P];
-    __shared__ float sw[MAX_P];
-    __shared__ unsigned rows[MAX_E];
-    __shared__ int jobof[MAX_E], wsum[MAX_P / WAVE];
-    for (int t = wave; t < T; t += NW) {
-        int pick;
-        float w;
-        topk_wave_e(logits + (size_t) t * (E + 1), E, K, lane, pick, w);
-        if (lane < K) {
-            ex[t * K + lane] = pick;
-            sw[t * K + lane] = w;
-        }
-    }
-    __syncthreads();
-    PickSlot ps;
-    const int nr = pick_slots(ex, P, K, rows, jobof, wsum, ps);
-    if (p < P) {
-        topi_g[p] = ex[p];
-        topw_g[p] = sw[p];
-        if (ps.e >= 0) {
-            const int j = ps.job;
-            if (ps.slot == 0) {
-                jg[j].w = jd[j].w = ps.e;
-                jg[j].n = jd[j].n = ps.cnt;
-            }
-            jg[j].y[ps.slot] = p / K;
-            jg[j].out[ps.slot] = jd[j].y[ps.slot] = jd[j].out[ps.slot] = p;
-        }
-    }
-    if (shared) {
-        if (p == 0) {
-            jg[nr].w = jd[nr].w = E;
-            jg[nr].n = jd[nr].n = T;
-        }
-        if (p < T) {
-            jg[nr].y[p] = p;
-            jg[nr].out[p] = jd[nr].y[p] = jd[nr].out[p] = P + p;
-        }
-    }
-    if (p == 0) {
-        njobs_g[0] = nr + (shared ? 1 : 0);
-        njobs_g[1] = 0;
-    }
-}
-
 // K2 for windows of several rows: a block is one (job, 32 FF indices) unit of the jobs K1b numbered, as at batch 1:
 // the first half of the waves take the 32 gate rows, the second half the matching up rows (a row a lane group, so a
 // lane holds one row's share), each dotted with the job's staged activation rows; SwiGLU and h as q8_1 per slot.

@@ -1,7 +1,7 @@
-// Activations and routing: q8_1 quantization, the decode router (logits, top-k, jobs in one launch), the prompt path's
+// Activations and routing: q8_1 quantization, the decode router (logits, then top-k and jobs), the prompt path's
 // router logits and permutation, and the weighted combine.
 #include "cache.hpp"
-#include "topk.hpp"
+#include "route_jobs.hpp"
 
 namespace sfnx {
 namespace {
@@ -33,115 +33,53 @@ __device__ __forceinline__ void row_load(const float* __restrict__ w, int lane, 
     for (int i = 0; i < NC; ++i) wv[i] = reinterpret_cast<const float4*>(w)[i * WAVE + lane];
 }
 template <int NC>
-__device__ __forceinline__ float row_dot(const float4 (&wv)[NC], const float* __restrict__ x, int lane) {
+__device__ __forceinline__ float row_dot(const float4 (&wv)[NC], const float4 (&xv)[NC]) {
     float a = 0.f;
 #pragma unroll
     for (int i = 0; i < NC; ++i) {
-        const float4 b = reinterpret_cast<const float4*>(x)[i * WAVE + lane];
-        a = fmaf(wv[i].x, b.x, a);
-        a = fmaf(wv[i].y, b.y, a);
-        a = fmaf(wv[i].z, b.z, a);
-        a = fmaf(wv[i].w, b.w, a);
+        a = fmaf(wv[i].x, xv[i].x, a);
+        a = fmaf(wv[i].y, xv[i].y, a);
+        a = fmaf(wv[i].z, xv[i].z, a);
+        a = fmaf(wv[i].w, xv[i].w, a);
     }
     return group_sum<WAVE>(a);
 }
 
 constexpr int RR_THREADS = 256, RR_WAVES = RR_THREADS / WAVE;
-// src/moe.cuh:73-202 k_router_route: the router's rows a wavefront each, the shared gate row E included; the last
-// block to finish takes the top-K of every token and builds the jobs (first-pick order, rows in pair order).  Returns
-// the job count in the last block, -1 in the others.
-template <int NC, int TT>
-__device__ __forceinline__ int router_route_body(const float* __restrict__ W, const float* __restrict__ x,
-                                                 float* __restrict__ logits, int T, int E, int K, int* __restrict__ topi,
-                                                 float* __restrict__ topw, sfnx_job* __restrict__ gu,
-                                                 sfnx_job* __restrict__ dn, int* __restrict__ njobs, int shared) {
+// src/moe.cuh:73-202 k_router_route as two launches, these logits (the shared gate row E included) and the routing in one
+// workgroup.  In one launch every block fenced its logits before the last block's top-k could read them; a kernel boundary
+// costs less.  A block takes one router row, its 4 wavefronts tokens g, g + 4, ... (one row a wavefront left 513 wavefronts,
+// two a compute unit, each with every token's chain in turn), the next token's chunks requested while one is summed.  Both
+// launches, 2048 columns and 513 router rows, against the one: 1 token 16.0 -> 8.8 us, 7 tokens 20.4 -> 9.9, 16 tokens
+// 27.8 -> 13.5; 2560 columns and 257 rows, 7 tokens: 15.9 -> 8.8.
+template <int NC>
+__global__ void __launch_bounds__(RR_THREADS) k_route_logits(const float* __restrict__ W, const float* __restrict__ x,
+                                                            float* __restrict__ logits, int T, int L) {
     constexpr int H = NC * 4 * WAVE;
-    const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE, L = E + 1;
-    const int row = blockIdx.x * RR_WAVES + wave;
-    if (row < L) {
-        float4 wv[NC];
-        row_load<NC>(W + (size_t) row * H, lane, wv);
-#pragma unroll
-        for (int t = 0; t < TT; ++t) {
-            if (t >= T) break;
-            const float s = row_dot<NC>(wv, x + (size_t) t * H, lane);
-            if (lane == 0) logits[(size_t) t * L + row] = s;
-        }
-    }
-    __shared__ int last;
-    __threadfence();
-    __syncthreads();
-    if (threadIdx.x == 0) last = atomicAdd(njobs + 1, 1) == (int) gridDim.x - 1;
-    __syncthreads();
-    if (!last) return -1;
-    __threadfence();
-    __shared__ int ex[MAX_P];
+    const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE, row = blockIdx.x;
+    if (wave >= T) return;
+    float4 wv[NC], xn[NC];
+    row_load<NC>(W + (size_t) row * H, lane, wv);
+    row_load<NC>(x + (size_t) wave * H, lane, xn);
     for (int t = wave; t < T; t += RR_WAVES) {
-        int pick;
-        float w;
-        topk_wave_e<true>(logits + (size_t) t * L, E, K, lane, pick, w);
-        if (lane < K) {
-            topi[t * K + lane] = pick;
-            topw[t * K + lane] = w;
-            ex[t * K + lane] = pick;
-        }
+        float4 xv[NC];
+#pragma unroll
+        for (int i = 0; i < NC; ++i) xv[i] = xn[i];
+        if (t + RR_WAVES < T) row_load<NC>(x + (size_t) (t + RR_WAVES) * H, lane, xn);
+        const float s = row_dot<NC>(wv, xv);
+        if (lane == 0) logits[(size_t) t * L + row] = s;
     }
-    __syncthreads();
-    // jobs: a job per distinct expert in first-pick order, rows in pair order
-    const int P = T * K;
-    __shared__ unsigned rows[MAX_E];
-    __shared__ int jobof[MAX_E], wsum[MAX_P / WAVE];
-    PickSlot ps;
-    const int nr = pick_slots(ex, P, K, rows, jobof, wsum, ps);
-    const int p = threadIdx.x;
-    if (p < P && ps.e >= 0) {
-        const int j = ps.job;
-        if (ps.slot == 0) {
-            gu[j].w = dn[j].w = ps.e;
-            gu[j].n = dn[j].n = ps.cnt;
-        }
-        gu[j].y[ps.slot] = p / K;
-        gu[j].out[ps.slot] = dn[j].y[ps.slot] = dn[j].out[ps.slot] = p;
-    }
-    const int nj = nr;
-    if (shared) {
-        if (p == 0) {
-            gu[nj].w = dn[nj].w = E;
-            gu[nj].n = dn[nj].n = T;
-        }
-        if (p < T) {
-            gu[nj].y[p] = p;
-            gu[nj].out[p] = dn[nj].y[p] = dn[nj].out[p] = P + p;
-        }
-    }
-    if (p == 0) {
-        njobs[0] = nj + (shared ? 1 : 0);
-        njobs[1] = 0;
-    }
-    return nj + (shared ? 1 : 0);
 }
 
-template <int NC, int TT>
-__global__ void __launch_bounds__(RR_THREADS) k_router_route(const float* __restrict__ W, const float* __restrict__ x,
-                                                            float* __restrict__ logits, int T, int E, int K,
-                                                            int* __restrict__ topi, float* __restrict__ topw,
-                                                            sfnx_job* __restrict__ gu, sfnx_job* __restrict__ dn,
-                                                            int* __restrict__ njobs, int shared) {
-    router_route_body<NC, TT>(W, x, logits, T, E, K, topi, topw, gu, dn, njobs, shared);
-}
-
-// The same with an expert cache: the last block's first wavefront then plans the window's slots for `layer`
-// (src/moe.cuh:128-198: the reference's router plans in its last block too), once the block's jobs are written, so a
-// cached layer takes no launch of its own for the plan.
-template <int NC, int TT>
-__global__ void __launch_bounds__(RR_THREADS) k_router_route_plan(const float* __restrict__ W, const float* __restrict__ x,
-                                                                 float* __restrict__ logits, int T, int E, int K,
-                                                                 int* __restrict__ topi, float* __restrict__ topw,
-                                                                 sfnx_job* __restrict__ gu, sfnx_job* __restrict__ dn,
-                                                                 int* __restrict__ njobs, int shared,
-                                                                 sfnx_expert_cache ec, int layer, int* __restrict__ list) {
-    const int nj = router_route_body<NC, TT>(W, x, logits, T, E, K, topi, topw, gu, dn, njobs, shared);
-    if (nj < 0) return;
+// The routing with an expert cache: the first wavefront then plans the window's slots for `layer` (src/moe.cuh:128-198: the
+// reference's router plans in its last block too), once the block's jobs are written, so a cached layer takes no launch of
+// its own for the plan.
+__global__ void __launch_bounds__(DR_THREADS) k_route_plan(int T, int E, int K, int shared, const float* __restrict__ logits,
+                                                           int* __restrict__ topi, float* __restrict__ topw,
+                                                           sfnx_job* __restrict__ gu, sfnx_job* __restrict__ dn,
+                                                           int* __restrict__ njobs, sfnx_expert_cache ec, int layer,
+                                                           int* __restrict__ list) {
+    const int nj = route_window(T, E, K, shared, logits, topi, topw, gu, dn, njobs);
     __syncthreads();   // every job of the block written
     if (threadIdx.x >= WAVE) return;
     plan_window(gu, nj, layer, ec, list, threadIdx.x, WaveSync{});
@@ -590,31 +528,15 @@ __global__ void __launch_bounds__(RN_THREADS) k_residual_rmsnorm(float* __restri
     for (int i = threadIdx.x; i < H; i += RN_THREADS) xn[(size_t) t * H + i] = xs[i] * rs;
 }
 
-template <int TT>
-void launch_router_tt(int nc, dim3 g, hipStream_t s, const float* W, const float* x, float* logits, int T, int E, int K,
-                      int* topi, float* topw, sfnx_job* gu, sfnx_job* dn, int* njobs, int shared) {
-    switch (nc) {
-        case 4: k_router_route<4, TT><<<g, RR_THREADS, 0, s>>>(W, x, logits, T, E, K, topi, topw, gu, dn, njobs, shared); break;
-        case 8: k_router_route<8, TT><<<g, RR_THREADS, 0, s>>>(W, x, logits, T, E, K, topi, topw, gu, dn, njobs, shared); break;
-        case 10: k_router_route<10, TT><<<g, RR_THREADS, 0, s>>>(W, x, logits, T, E, K, topi, topw, gu, dn, njobs, shared); break;
-        case 16: k_router_route<16, TT><<<g, RR_THREADS, 0, s>>>(W, x, logits, T, E, K, topi, topw, gu, dn, njobs, shared); break;
+void launch_route_logits(hipStream_t s, const float* W, const float* x, float* logits, int T, int H, int L) {
+    switch (H / 256) {
+        case 4: k_route_logits<4><<<L, RR_THREADS, 0, s>>>(W, x, logits, T, L); break;
+        case 8: k_route_logits<8><<<L, RR_THREADS, 0, s>>>(W, x, logits, T, L); break;
+        case 10: k_route_logits<10><<<L, RR_THREADS, 0, s>>>(W, x, logits, T, L); break;
+        case 16: k_route_logits<16><<<L, RR_THREADS, 0, s>>>(W, x, logits, T, L); break;
         default: throw std::runtime_error("hidden size must be 1024, 2048, 2560 or 4096");
     }
-}
-
-template <int TT>
-void launch_router_plan_tt(int nc, dim3 g, hipStream_t s, const float* W, const float* x, float* logits, int T, int E,
-                           int K, int* topi, float* topw, sfnx_job* gu, sfnx_job* dn, int* njobs, int shared,
-                           const sfnx_expert_cache& ec, int layer, int* list) {
-#define SFNX_RRP(NCV) k_router_route_plan<NCV, TT><<<g, RR_THREADS, 0, s>>>(W, x, logits, T, E, K, topi, topw, gu, dn, njobs, shared, ec, layer, list)
-    switch (nc) {
-        case 4: SFNX_RRP(4); break;
-        case 8: SFNX_RRP(8); break;
-        case 10: SFNX_RRP(10); break;
-        case 16: SFNX_RRP(16); break;
-        default: throw std::runtime_error("hidden size must be 1024, 2048, 2560 or 4096");
-    }
-#undef SFNX_RRP
+    check(hipGetLastError(), "k_route_logits launch");
 }
 
 }  // namespace
@@ -638,12 +560,9 @@ extern "C" int sfnx_router_route(const float* W, const float* x, float* logits, 
         require(E >= WAVE && E % WAVE == 0 && E <= MAX_E, "E must be a multiple of 64, at most 1024");
         require(K >= 1 && K <= MAX_K && K <= E, "K out of range (1..16)");
         require(H % 256 == 0, "H must be a multiple of 256");
-        const dim3 g((E + 1 + RR_WAVES - 1) / RR_WAVES);
-        const int nc = H / 256;
         hipStream_t s = stream_of(st);
-        if (T == 1) launch_router_tt<1>(nc, g, s, W, x, logits, T, E, K, topi, topw, jobs_gu, jobs_dn, njobs, shared);
-        else if (T <= 4) launch_router_tt<4>(nc, g, s, W, x, logits, T, E, K, topi, topw, jobs_gu, jobs_dn, njobs, shared);
-        else launch_router_tt<16>(nc, g, s, W, x, logits, T, E, K, topi, topw, jobs_gu, jobs_dn, njobs, shared);
+        launch_route_logits(s, W, x, logits, T, H, E + 1);
+        k_dec_route<<<1, DR_THREADS, 0, s>>>(T, E, K, shared, logits, topi, topw, jobs_gu, jobs_dn, njobs);
     });
 }
 
@@ -659,12 +578,9 @@ extern "C" int sfnx_router_route_plan(const float* W, const float* x, float* log
         check_cache(ec);
         check_layer(ec, layer);
         require(E + (shared ? 1 : 0) <= ec->n_experts, "the layer's experts (and its shared expert) pass the cache's tables");
-        const dim3 g((E + 1 + RR_WAVES - 1) / RR_WAVES);
-        const int nc = H / 256;
         hipStream_t s = stream_of(st);
-        if (T == 1) launch_router_plan_tt<1>(nc, g, s, W, x, logits, T, E, K, topi, topw, jobs_gu, jobs_dn, njobs, shared, *ec, layer, list);
-        else if (T <= 4) launch_router_plan_tt<4>(nc, g, s, W, x, logits, T, E, K, topi, topw, jobs_gu, jobs_dn, njobs, shared, *ec, layer, list);
-        else launch_router_plan_tt<16>(nc, g, s, W, x, logits, T, E, K, topi, topw, jobs_gu, jobs_dn, njobs, shared, *ec, layer, list);
+        launch_route_logits(s, W, x, logits, T, H, E + 1);
+        k_route_plan<<<1, DR_THREADS, 0, s>>>(T, E, K, shared, logits, topi, topw, jobs_gu, jobs_dn, njobs, *ec, layer, list);
     });
 }
 

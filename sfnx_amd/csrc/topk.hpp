@@ -85,10 +85,10 @@ __device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
 }
 
 // one token's E = 64 NV logits into registers, lane l holding experts l + 64 i (i < nv; the rest NaN)
-template <int NV, bool AGENT = false>
+template <int NV>
 __device__ __forceinline__ void topk_load(const float* lg, int nv, int lane, float (&lv)[NV]) {
 #pragma unroll
-    for (int i = 0; i < NV; ++i) lv[i] = i >= nv ? NAN : AGENT ? load_agent(lg + lane + WAVE * i) : lg[lane + WAVE * i];
+    for (int i = 0; i < NV; ++i) lv[i] = i >= nv ? NAN : lg[lane + WAVE * i];
 }
 
 // The top-K of one token's logits (lane l holds experts l + 64 i) by one wavefront: K rounds of the largest untaken
@@ -214,22 +214,20 @@ __device__ inline void topk_core(const float (&lv)[NV], int K, int lane, int& pi
     weight = topk_weight(pick, po, K);
 }
 
-// AGENT: the logits were written earlier in the same launch
-template <int NV, bool AGENT = false>
+template <int NV>
 __device__ inline void topk_wave(const float* lg, int nv, int K, int lane, int& pick, float& weight) {
     float lv[NV];
-    topk_load<NV, AGENT>(lg, nv, lane, lv);
+    topk_load<NV>(lg, nv, lane, lv);
     topk_core<NV>(lv, K, lane, pick, weight);
 }
 // E at run time (a multiple of 64, at most 1024): the smallest instantiation that holds E / 64 values a lane
-template <bool AGENT = false>
 __device__ inline void topk_wave_e(const float* lg, int E, int K, int lane, int& pick, float& weight) {
     const int nv = E / WAVE;
-    if (nv <= 1) topk_wave<1, AGENT>(lg, nv, K, lane, pick, weight);
-    else if (nv <= 2) topk_wave<2, AGENT>(lg, nv, K, lane, pick, weight);
-    else if (nv <= 4) topk_wave<4, AGENT>(lg, nv, K, lane, pick, weight);
-    else if (nv <= 8) topk_wave<8, AGENT>(lg, nv, K, lane, pick, weight);
-    else topk_wave<16, AGENT>(lg, nv, K, lane, pick, weight);
+    if (nv <= 1) topk_wave<1>(lg, nv, K, lane, pick, weight);
+    else if (nv <= 2) topk_wave<2>(lg, nv, K, lane, pick, weight);
+    else if (nv <= 4) topk_wave<4>(lg, nv, K, lane, pick, weight);
+    else if (nv <= 8) topk_wave<8>(lg, nv, K, lane, pick, weight);
+    else topk_wave<16>(lg, nv, K, lane, pick, weight);
 }
 
 // Decode jobs (src/moe.cuh:164-198, tools/kbench.cu:77-95): one job per distinct expert numbered in the order of each

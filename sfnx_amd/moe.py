@@ -61,8 +61,8 @@ def quantize_q8_1(x: torch.Tensor, q: torch.Tensor) -> None:
 
 def router_route(W, x, logits, topi, topw, jobs_gu, jobs_dn, njobs, E: int, K: int, shared: bool = True,
                  plan=None) -> None:
-    """src/kernels.hpp:269-278 router_route; plan = (cache, layer, list): the same launch's last block also plans the
-    window's slots in the ExpertCache (sfnx_router_route_plan)"""
+    """src/kernels.hpp:269-278 router_route; plan = (cache, layer, list): the routing launch also plans the window's
+    slots in the ExpertCache (sfnx_router_route_plan)"""
     T, H = x.shape
     if plan is None:
         check(lib().sfnx_router_route(_p(W), _p(x), _p(logits), T, H, E, K, _p(topi), _p(topw), _p(jobs_gu),
@@ -707,7 +707,7 @@ class ExpertCache:
 def decode_layer_cached(cache: ExpertCache, l: int, x: torch.Tensor, y: torch.Tensor, b: DecodeBuffers, out_list,
                         plan_in_router: bool = True) -> None:
     """decode_layer with the layer's experts behind the expert cache (src/engine.cu:947-971): the routing with the
-    window's slots planned in its last block (or, plan_in_router=False, the plan as a launch of its own), the planned
+    window's slots planned in its launch (or, plan_in_router=False, the plan as a launch of its own), the planned
     experts copied in (moe_cache), then the expert calls through the layer's tables"""
     V = cache.layer_view(l)
     s = V.s

@@ -61,6 +61,16 @@ def test_router_route_random(T, shared):
     route_case(W, x, E, K, shared)
 
 
+@pytest.mark.parametrize("T, H, E, K", [(1, 1024, 64, 1), (3, 4096, 64, 16), (4, 2560, 1024, 10), (9, 1024, 128, 6),
+                                        (13, 4096, 1024, 16), (16, 2560, 64, 16)])
+def test_router_route_edges(T, H, E, K):
+    """windows that leave some of a block's four wavefronts a token less than others, every hidden size, few and many
+    experts; the shared job on odd T"""
+    W = orc.synth((E + 1) * H, 220 + T, 0.02).reshape(E + 1, H)
+    x = orc.synth(T * H, 221 + T, 1.0).reshape(T, H)
+    route_case(W, x, E, K, bool(T % 2))
+
+
 def test_router_route_exact_ties():
     """duplicated router rows give exactly equal logits: the lower expert wins, as in tools/topk_test.cu"""
     H, E, K = 2048, 512, 10
