@@ -17,6 +17,15 @@ namespace {
 constexpr int MV_THREADS = 256;
 
 // ------------------------------------------------------------------------------------------------ the kernel
+// Row tiles (256 / lanes a row) a block.  A block of down makes its rows' h itself (silu and the quantization, ~45
+// instructions a value), so two tiles, requested together before it, halve that work: a block is 32 rows in every type, the
+// K-quants' 8 lanes a row reaching that with one tile.  Down, 512 columns, 512 experts, top 10 plus the shared one, with
+// weights from HBM: Q8_0 33.6 -> 28.9 us at 7 rows, 62 -> 50.4 at 16; Q5_1 34.6 -> 26.8, 65 -> 44.4; 1024 columns, 256
+// experts: Q8_0 99 -> 81 at 16.  Three and four tiles lost part of it again, K-quants with two took 10% more, and gate|up,
+// whose staging is a copy, gained nothing (Q8_0 71 -> 74).  Past 2048 columns two tiles' rows fill the registers.
+template <int TYPE, int G, bool DOWN> __host__ __device__ constexpr int mv_tiles() {
+    return DOWN && !is_kquant(TYPE) && G <= 4 ? 2 : 1;
+}
 // TYPE: SFNX_Q4_K / SFNX_Q5_K (8 lanes a row) or SFNX_Q8_0 (16 lanes a row); G: groups or blocks per lane = C / 512;
 // TT: activation rows per pass; DOWN: activations from gu rows through swiglu (else q8_1 rows).
 template <int TYPE, int G, int TT, bool DOWN>
@@ -33,33 +42,46 @@ k_moe_mv(const uint8_t* __restrict__ A, size_t sa, int R, int C, const sfnx_job*
     __shared__ sfnx_job jb;
     load_job(jb, jobs + ji);
     __syncthreads();
-    const int row = blockIdx.x * RPB + threadIdx.x / LPR, ln = threadIdx.x % LPR;
-    const bool live = row < R;
+    constexpr int NTL = mv_tiles<TYPE, G, DOWN>();
+    const int r0 = blockIdx.x * NTL * RPB + threadIdx.x / LPR, ln = threadIdx.x % LPR;
     const Acts a = acts_in(lds, TT, C);
-    typename RowOf<TYPE, G>::R w;
-    if (live) RowOf<TYPE, G>::load(w, expert_at(A, sa, jb.w), R, row, C, ln);
+    const uint8_t* mat = expert_at(A, sa, jb.w);
+    typename RowOf<TYPE, G>::R w[NTL];
+#pragma unroll
+    for (int i = 0; i < NTL; ++i)
+        if (r0 + i * RPB < R) RowOf<TYPE, G>::load(w[i], mat, R, r0 + i * RPB, C, ln);
     for (int j0 = 0; j0 < jb.n; j0 += TT) {
         const int nn = min(TT, jb.n - j0);
         if (j0) __syncthreads();
         if constexpr (DOWN) stage_swiglu(a, (const float*) in, jb.y + j0, nn);
         else stage_q8_1(a, (const uint8_t*) in, jb.y + j0, nn);
         __syncthreads();
-        for (int j = 0; j < nn; ++j) {
-            const float v = group_sum<LPR>(live ? w.dot(a, j, ln) : 0.f);
-            if (live && ln == 0) out[(size_t) jb.out[j0 + j] * R + row] = v;
-        }
+        for (int j = 0; j < nn; ++j)
+#pragma unroll
+            for (int i = 0; i < NTL; ++i) {
+                const bool live = r0 + i * RPB < R;
+                const float v = group_sum<LPR>(live ? w[i].dot(a, j, ln) : 0.f);
+                if (live && ln == 0) out[(size_t) jb.out[j0 + j] * R + r0 + i * RPB] = v;
+            }
     }
 }
 
+template <int TYPE, int G, int TT, bool DOWN>
+void launch_mv(int njobs_max, size_t lds, hipStream_t s, const uint8_t* A, size_t sa, int R, int C, const sfnx_job* jobs,
+               const int* njobs, const void* in, float* out) {
+    constexpr int rows = MV_THREADS / lpr_of<TYPE>() * mv_tiles<TYPE, G, DOWN>();
+    k_moe_mv<TYPE, G, TT, DOWN><<<dim3((R + rows - 1) / rows, njobs_max), MV_THREADS, lds, s>>>(A, sa, R, C, jobs, njobs, in, out);
+}
+
 template <int TYPE, int TT, bool DOWN>
-void launch_g(int G, dim3 grid, size_t lds, hipStream_t s, const uint8_t* A, size_t sa, int R, int C, const sfnx_job* jobs,
+void launch_g(int G, int njobs_max, size_t lds, hipStream_t s, const uint8_t* A, size_t sa, int R, int C, const sfnx_job* jobs,
               const int* njobs, const void* in, float* out) {
     switch (G) {
-        case 1: k_moe_mv<TYPE, 1, TT, DOWN><<<grid, MV_THREADS, lds, s>>>(A, sa, R, C, jobs, njobs, in, out); break;
-        case 2: k_moe_mv<TYPE, 2, TT, DOWN><<<grid, MV_THREADS, lds, s>>>(A, sa, R, C, jobs, njobs, in, out); break;
-        case 4: k_moe_mv<TYPE, 4, TT, DOWN><<<grid, MV_THREADS, lds, s>>>(A, sa, R, C, jobs, njobs, in, out); break;
-        case 5: k_moe_mv<TYPE, 5, TT, DOWN><<<grid, MV_THREADS, lds, s>>>(A, sa, R, C, jobs, njobs, in, out); break;
-        case 8: k_moe_mv<TYPE, 8, TT, DOWN><<<grid, MV_THREADS, lds, s>>>(A, sa, R, C, jobs, njobs, in, out); break;
+        case 1: launch_mv<TYPE, 1, TT, DOWN>(njobs_max, lds, s, A, sa, R, C, jobs, njobs, in, out); break;
+        case 2: launch_mv<TYPE, 2, TT, DOWN>(njobs_max, lds, s, A, sa, R, C, jobs, njobs, in, out); break;
+        case 4: launch_mv<TYPE, 4, TT, DOWN>(njobs_max, lds, s, A, sa, R, C, jobs, njobs, in, out); break;
+        case 5: launch_mv<TYPE, 5, TT, DOWN>(njobs_max, lds, s, A, sa, R, C, jobs, njobs, in, out); break;
+        case 8: launch_mv<TYPE, 8, TT, DOWN>(njobs_max, lds, s, A, sa, R, C, jobs, njobs, in, out); break;
         default: throw std::runtime_error("input width must be 512, 1024, 2048, 2560 or 4096");
     }
 }
@@ -79,11 +101,9 @@ void moe_mv(uint32_t type, const void* A, size_t sa, int n_in, int n_out, const 
     if (acts_bytes(TT, n_in) > 64 * 1024) TT = 4;
     const size_t lds = acts_bytes(TT, n_in);
     require(lds <= 64 * 1024, "activation rows do not fit the LDS budget");
-    const int rpb = MV_THREADS / (is_kquant(type) ? 8 : 16);
-    const dim3 grid((n_out + rpb - 1) / rpb, njobs_max);
     hipStream_t s = stream_of(st);
     const uint8_t* a = (const uint8_t*) A;
-#define SFNX_MV(TY, TTV) launch_g<TY, TTV, DOWN>(G, grid, lds, s, a, sa, n_out, n_in, jobs, njobs, in, out)
+#define SFNX_MV(TY, TTV) launch_g<TY, TTV, DOWN>(G, njobs_max, lds, s, a, sa, n_out, n_in, jobs, njobs, in, out)
     if (type == SFNX_Q4_K) {
         if (TT == 1) SFNX_MV(SFNX_Q4_K, 1);
         else if (TT == 4) SFNX_MV(SFNX_Q4_K, 4);

@@ -82,3 +82,10 @@ def test_bigjobs_none(wtype):
     x = torch.zeros((4, 1024), device="cuda")
     moe.moe_down_big(A, 128 * moe.row_bytes(wtype, 512), wtype, 512, 128, jobs, n0, 2, x, out)
     assert torch.all(out == 7.0)
+
+
+@pytest.mark.parametrize("wtype", TYPES)
+@pytest.mark.parametrize("n_in, n_out", [(512, 32), (1024, 64), (2048, 32)])
+def test_down_few_rows(wtype, n_in, n_out):
+    """the fewest rows a store holds: one or two window blocks of two row tiles"""
+    test_bigjobs_equal_windows(wtype, n_in, n_out, True)
