@@ -229,14 +229,16 @@ __device__ __forceinline__ void dequant_step(const Chunk<SFNX_Q5_K>& w, int s, h
     deq_q4k(w.q[s], half2v{D[0], D[0]}, half2v{N[0], N[0]}, half2v{D[1], D[1]}, half2v{N[1], N[1]}, b, &w.qh, 2 * s);
 }
 // Q4_0 / Q5_1: a block's 16 quant bytes (value l in the low nibble of byte l, l + 16 in the high) -> the 4 B
-// fragments, fragment c holding values 8 c .. 8 c + 7; Q4_0 hmul2(q - 8, d), as hfma2(q, d, -8 d) (-8 d is exact, so the one
-// rounding is of the same product), Q5_1 hfma2(q, d, m) with the fifth bits
+// fragments, fragment c holding values 8 c .. 8 c + 7; Q4_0 hmul2(q - 8, d), Q5_1 hfma2(q, d, m) with the fifth bits.
+// (Q4_0 as hfma2(q, d, -8 d) is an instruction less a pair and measured 188 us for 198 in the gate|up of 2048 tokens, but
+// -8 d leaves f16 past |d| = 8188, where the products of the values about 8 are still finite.  A branch to this form for
+// such blocks measured 205.)
 template <int TYPE>
 __device__ __forceinline__ void deq_nb(const uint4& q, uint32_t dm, uint32_t qh, half8 (&b)[4]) {
     const uint32_t w[4] = {q.x, q.y, q.z, q.w};
     const half2v d = {__builtin_bit_cast(_Float16, (uint16_t) (dm & 0xffff)), __builtin_bit_cast(_Float16, (uint16_t) (dm & 0xffff))};
-    const half2v k1024 = {(_Float16) 1024.0f, (_Float16) 1024.0f}, m8 = {(_Float16) -8.0f, (_Float16) -8.0f};
-    const half2v m = TYPE == SFNX_Q4_0 ? d * m8 : half2v{__builtin_bit_cast(_Float16, (uint16_t) (dm >> 16)), __builtin_bit_cast(_Float16, (uint16_t) (dm >> 16))};
+    const half2v m = {__builtin_bit_cast(_Float16, (uint16_t) (dm >> 16)), __builtin_bit_cast(_Float16, (uint16_t) (dm >> 16))};
+    const half2v k1024 = {(_Float16) 1024.0f, (_Float16) 1024.0f}, k8 = {(_Float16) 8.0f, (_Float16) 8.0f};
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
         const bool hi = c >= 2;
@@ -245,9 +247,14 @@ __device__ __forceinline__ void deq_nb(const uint4& q, uint32_t dm, uint32_t qh,
             const int wi = 2 * (c % 2) + p;   // the dword: values 4 wi .. 4 wi + 3 (+ 16 for the high nibbles)
             uint32_t v = hi ? (w[wi] >> 4) & 0x0F0F0F0Fu : w[wi] & 0x0F0F0F0Fu;
             if constexpr (TYPE == SFNX_Q5_1) v |= spread4(qh >> ((hi ? 16 : 0) + 4 * wi));
-            const half2v q01 = TYPE == SFNX_Q4_0 ? nibbles_f16<0>(v) : bytes_1024<0>(v) - k1024;
-            const half2v q23 = TYPE == SFNX_Q4_0 ? nibbles_f16<1>(v) : bytes_1024<1>(v) - k1024;
-            const half2v r01 = __builtin_elementwise_fma(q01, d, m), r23 = __builtin_elementwise_fma(q23, d, m);
+            half2v r01, r23;
+            if constexpr (TYPE == SFNX_Q4_0) {
+                r01 = (nibbles_f16<0>(v) - k8) * d;
+                r23 = (nibbles_f16<1>(v) - k8) * d;
+            } else {
+                r01 = __builtin_elementwise_fma(bytes_1024<0>(v) - k1024, d, m);
+                r23 = __builtin_elementwise_fma(bytes_1024<1>(v) - k1024, d, m);
+            }
             b[c][4 * p + 0] = r01[0];
             b[c][4 * p + 1] = r01[1];
             b[c][4 * p + 2] = r23[0];

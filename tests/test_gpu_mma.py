@@ -285,3 +285,33 @@ def test_mma_wide_hidden(H, ff, wtype):
     assert np.array_equal(b.topi.cpu().numpy(), oi)
     eg, ed = check_sampled(host, x, b, 24, np.random.default_rng(H))
     assert eg < 2e-3 and ed < 2e-3, (eg, ed)
+
+
+@pytest.mark.parametrize("C", [512, 1024])   # the two kernels of moe_gate_up_mma
+def test_q4_0_largest_scales(C):
+    """Q4_0 blocks of any finite f16 scale: (q - 8) d is finite wherever the product is, at scales about 8188 (where 8 d
+    leaves f16), at the largest, and in both signs; against the oracle's f16 weights.  512 or 1024 products in fp32: an error
+    of at most about 1024 x 2^-24 of the sum of their magnitudes in the worst order, 1e-5 of the largest sum in practice"""
+    R, rng = 512, np.random.default_rng(8)
+    d = np.array([1.0, 8188, 8192, 9000, 16384, 21824, 32768, 65504], np.float16)
+    g = np.zeros((R, C // 32, 18), np.uint8)
+    dd = d[rng.integers(0, d.size, (R, C // 32))] * np.where(rng.random((R, C // 32)) < 0.5, -1, 1).astype(np.float16)
+    g[:, :, :2] = dd.view(np.uint8).reshape(R, C // 32, 2)
+    top = np.floor(65504 / np.abs(dd.astype(np.float64))).clip(max=7).astype(int)[..., None]   # |q - 8| that stay finite
+    q = rng.integers(-top, top + 1, (R, C // 32, 32)) + 8
+    g[:, :, 2:] = (q[..., :16] | (q[..., 16:] << 4)).astype(np.uint8)
+    w = orc.dequant_f16(orc.Q4_0, g.reshape(-1), R, C).view(np.float16).astype(np.float64).reshape(R, C)
+    assert np.isfinite(w).all() and np.abs(w).max() > 60000
+    src = torch.from_numpy(g.reshape(-1)).cuda()
+    A = torch.empty_like(src)
+    moe.store_pack(orc.Q4_0, src, A, 1, R, C)
+    job = np.zeros((1, orc.BIGJOB_DTYPE.itemsize // 4), np.int32)
+    job[0, 1] = 5
+    job[0, 2:7] = job[0, 66:71] = np.arange(5)
+    jobs, nj = torch.from_numpy(job).cuda(), torch.tensor([1, 0], dtype=torch.int32, device="cuda")
+    x = (rng.standard_normal((5, C)) * 2.0 ** -10).astype(np.float16)
+    out = torch.zeros((5, R), device="cuda")
+    moe.moe_gate_up_mma(A, R * moe.row_bytes(orc.Q4_0, C), orc.Q4_0, C, R, jobs, nj, 1, torch.from_numpy(x).cuda(), out)
+    torch.cuda.synchronize()
+    want = x.astype(np.float64) @ w.T
+    assert max_rel(out.cpu().numpy(), want) < 1e-5
