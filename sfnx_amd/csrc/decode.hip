@@ -652,9 +652,12 @@ void launch_k3(const DecArgs& d, const sfnx_moe_layer_w& w, float* x, const DecL
     }
     const int NP = d.T * d.K + d.T;
     const size_t job_lds = d3_jobs_bytes(d.T * d.K + (d.shared ? 1 : 0)), hq_lds = job_lds + acts_bytes(NP, d.ff);
-    // every pair's h in LDS when it fits beside the jobs and the kernel's own ~12 KB (160 KB a workgroup on gfx950; past
-    // 64 KB the kernel must be allowed the larger dynamic size first), else read from L2 per task
-    constexpr size_t DYN_MAX = 144 * 1024;
+    // every pair's h in LDS when it fits beside the jobs and the kernel's own 11.1 KB (160 KB a workgroup on gfx950; past
+    // 64 KB the kernel must be allowed the larger dynamic size first), else read from L2 per task.  148 KB holds every
+    // window whose h is at most 120 KB, whatever its jobs (12 rows of 15 picks, FF 512, Q4_K: staged 21.3 us, from L2 30.7)
+    constexpr size_t DYN_MAX = 148 * 1024;
+    static_assert(acts_bytes(192, 512) == 120 * 1024 && d3_jobs_bytes(12 * 15 + 1) + acts_bytes(192, 512) <= DYN_MAX &&
+                  d3_jobs_bytes(11 * 16 + 1) + acts_bytes(11 * 17, 512) <= DYN_MAX);
     // 1024 threads (4 wavefronts a SIMD: the per-pair dot chains are latency-bound) where 128 registers hold a lane's
     // tasks (FF 512; not Q5_K, whose rows carry their fifth bits)
     constexpr int NT = G2 == 1 && TYPE != SFNX_Q5_K ? 1024 : 512;

@@ -32,7 +32,7 @@ __device__ __forceinline__ Acts acts_in(unsigned char* lds, int TT, int K) {
     a.K = K;
     return a;
 }
-__host__ __device__ inline size_t acts_bytes(int TT, int K) { return (size_t) TT * K + (size_t) TT * (K / 32) * 8; }
+__host__ __device__ constexpr size_t acts_bytes(int TT, int K) { return (size_t) TT * K + (size_t) TT * (K / 32) * 8; }
 
 // rows ys[0..n) (rows 0..n-1 when ys is null) of q8_1 activations (36-byte blocks) into LDS: a thread per (row, block)
 __device__ inline void stage_q8_1(const Acts& a, const uint8_t* __restrict__ xq, const int* ys, int n) {

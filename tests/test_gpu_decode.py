@@ -119,11 +119,12 @@ def test_mixed_gate_up_and_down_types(wtype, dn_type):
 @pytest.mark.parametrize("H, E, K, ff, wtype, T", [
     (2560, 1024, 16, 1024, orc.Q4_K, 1), (2560, 1024, 16, 1024, orc.Q4_K, 4), (4096, 128, 4, 512, orc.Q5_K, 1),
     (4096, 128, 4, 512, orc.Q8_0, 16), (1024, 1024, 1, 1024, orc.Q4_0, 2), (2560, 256, 8, 512, orc.Q5_1, 16),
-    (2048, 512, 10, 1024, orc.Q4_K, 16)])
+    (2048, 512, 10, 1024, orc.Q4_K, 16), (2048, 256, 15, 512, orc.Q4_K, 12), (1024, 64, 16, 512, orc.Q8_0, 11)])
 def test_fused_decode_edge_shapes(H, E, K, ff, wtype, T):
     """the fused decode's limits: hidden 2560 and 4096, 1024 experts, top-16 and top-1, FF 1024, windows of 1 to 16
-    rows: equal to the unfused path bit for bit and to the oracle within 2e-3.  The last case's h (176 pairs of 1024)
-    does not fit in the down kernel's LDS, so its down dots read h from memory (the unstaged branch)."""
+    rows: equal to the unfused path bit for bit and to the oracle within 2e-3.  The h of 176 pairs of 1024
+    does not fit in the down kernel's LDS, so its down dots read h from memory (the unstaged branch); the h of 12 rows of
+    15 picks (and of 11 of 16) at FF 512 fills it beside the window's jobs."""
     shape = moe.LayerShape(H=H, E=E, K=K, ff=ff, wtype=wtype, shared=True)
     L, host = make_layer(shape, 70 + H % 97 + K)
     x0 = torch.from_numpy(orc.synth(T * H, 830 + T + K, 1.0).reshape(T, H)).cuda()
