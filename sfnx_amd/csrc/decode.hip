@@ -110,6 +110,14 @@ __global__ void __launch_bounds__(D1_THREADS * d1_groups<TT>()) k_dec_router(con
 }
 
 // ------------------------------------------------------------------------------------------------ K2
+// K-quant rows kept packed across a job's rows (most jobs hold one or two): the nibbles split anew for each cost less than
+// the registers of a split row where those registers cost workgroups a compute unit.  Q4_K at 2048 columns 128 -> 75
+// registers, three workgroups: 38.8 -> 34.9 us at 16 rows; Q5_K at 2560 columns 150 -> 126, two: 42.0 -> 34.5 us at 5 rows.
+// Elsewhere they buy none, or none that pays, and packed rows took longer: 12 rows at 1024 columns Q5_K 17.0 -> 25.0 us,
+// Q4_K 17.0 -> 18.6; at 4096 columns 55.8 -> 62.5 and 43.8 -> 45.6; Q5_K at 2048 columns, 3 rows, 17.0 -> 18.6.
+template <int TYPE, int G> constexpr bool d2_packed() {
+    return (TYPE == SFNX_Q4_K && (G == 4 || G == 5)) || (TYPE == SFNX_Q5_K && G == 5);
+}
 // K2 for windows of several rows: a block is one (job, 32 FF indices) unit of the jobs K1b numbered, as at batch 1:
 // the first half of the waves take the 32 gate rows, the second half the matching up rows (a row a lane group, so a
 // lane holds one row's share), each dotted with the job's staged activation rows; SwiGLU and h as q8_1 per slot.
@@ -159,11 +167,8 @@ __global__ void __launch_bounds__(2 * d2_threads<TYPE>()) k_dec_experts(
         const Q8sPlanes Ps = sh_gu;
         for (int s = 0; s < jb.n; ++s) put(s, group_sum<LPR>(q8s_dot<LPR>(Ps, row, H, ln, a, s)));
     } else {
-        // (most jobs hold one or two rows: the nibbles split anew for each cost less than the registers of a split row.
-        // Q4_K at 2048 columns 128 -> 75 registers, three workgroups a compute unit: 38.8 -> 34.9 us at 16 rows; Q5_K at
-        // 2560 columns 150 -> 126, two: 42.0 -> 34.5 us at 5 rows)
         for (int s = 0; s < jb.n; ++s) {
-            if constexpr (is_kquant(TYPE)) w.pin();
+            if constexpr (d2_packed<TYPE, G>()) w.pin();
             put(s, group_sum<LPR>(w.dot(a, s, ln)));
         }
     }

@@ -119,7 +119,8 @@ def test_mixed_gate_up_and_down_types(wtype, dn_type):
 @pytest.mark.parametrize("H, E, K, ff, wtype, T", [
     (2560, 1024, 16, 1024, orc.Q4_K, 1), (2560, 1024, 16, 1024, orc.Q4_K, 4), (4096, 128, 4, 512, orc.Q5_K, 1),
     (4096, 128, 4, 512, orc.Q8_0, 16), (1024, 1024, 1, 1024, orc.Q4_0, 2), (2560, 256, 8, 512, orc.Q5_1, 16),
-    (2048, 512, 10, 1024, orc.Q4_K, 16), (2048, 256, 15, 512, orc.Q4_K, 12), (1024, 64, 16, 512, orc.Q8_0, 11)])
+    (2048, 512, 10, 1024, orc.Q4_K, 16), (2048, 256, 15, 512, orc.Q4_K, 12), (1024, 64, 16, 512, orc.Q8_0, 11),
+    (1024, 64, 6, 512, orc.Q5_K, 12), (4096, 64, 3, 512, orc.Q5_K, 5), (4096, 64, 3, 512, orc.Q4_K, 12), (2560, 64, 8, 512, orc.Q5_K, 3)])
 def test_fused_decode_edge_shapes(H, E, K, ff, wtype, T):
     """the fused decode's limits: hidden 2560 and 4096, 1024 experts, top-16 and top-1, FF 1024, windows of 1 to 16
     rows: equal to the unfused path bit for bit and to the oracle within 2e-3.  The h of 176 pairs of 1024
