@@ -118,11 +118,15 @@ __global__ void __launch_bounds__(D1_THREADS * d1_groups<TT>()) k_dec_router(con
 template <int TYPE, int G> constexpr bool d2_packed() {
     return (TYPE == SFNX_Q4_K && (G == 4 || G == 5)) || (TYPE == SFNX_Q5_K && G == 5);
 }
+// Wavefronts a SIMD the 16-lane types' kernels are held to (8: two 1024-thread workgroups a compute unit, 64 registers), where
+// they come near it by themselves: at 2048 columns Q8_0 had 67 and Q5_1 65, so one workgroup; 16 rows 60.8 -> 57.6 and
+// 56.0 -> 48.9 us
+template <int TYPE, int G> constexpr int d2_simd_waves() { return !is_kquant(TYPE) && G <= 4 ? 8 : 1; }
 // K2 for windows of several rows: a block is one (job, 32 FF indices) unit of the jobs K1b numbered, as at batch 1:
 // the first half of the waves take the 32 gate rows, the second half the matching up rows (a row a lane group, so a
 // lane holds one row's share), each dotted with the job's staged activation rows; SwiGLU and h as q8_1 per slot.
 template <int TYPE, int G, int TT>
-__global__ void __launch_bounds__(2 * d2_threads<TYPE>()) k_dec_experts(
+__global__ void __launch_bounds__(2 * d2_threads<TYPE>(), (d2_simd_waves<TYPE, G>())) k_dec_experts(
     const uint8_t* __restrict__ A, size_t sa, int H, int E, int ff, const uint8_t* __restrict__ xq,
     const sfnx_job* __restrict__ jg, const int* __restrict__ njobs_g, float* __restrict__ gu, int8_t* __restrict__ hq_q,
     float* __restrict__ hq_d, int* __restrict__ hq_s, Q8sPlanes sh_gu) {

@@ -42,3 +42,12 @@ def test_decode_kernels_do_not_spill(kernels):
     dec = {n: v for n, v in kernels.items() if "k_dec_" in n or "k_moe_mv" in n or "k_route" in n}
     assert len(dec) > 100
     assert not {n: v for n, v in dec.items() if v[1]}
+
+
+@pytest.mark.parametrize("wtype", [2, 7, 8])
+@pytest.mark.parametrize("G", [2, 4])
+def test_window_gate_up_two_workgroups(kernels, wtype, G):
+    """the windows' gate|up of the 32-value types up to 2048 columns: 1024-thread workgroups, two a compute unit in 64
+    registers"""
+    v = [v[0] for n, v in kernels.items() if f"k_dec_expertsILi{wtype}ELi{G}E" in n]
+    assert v and max(v) <= 64
