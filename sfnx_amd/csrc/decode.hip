@@ -362,7 +362,7 @@ __global__ void __launch_bounds__(NT, NT == 512 && is_kquant(TYPE) ? 2 : 4) k_de
     const bool staged = hq_in_lds != 0;
     const int g = threadIdx.x / LPR, ln = threadIdx.x % LPR;
     // with its own dense Q8_0 matrix the shared expert's job (the last) runs apart, in the reference's q8s sums
-    const int nq = sh_dn.q != nullptr && shared ? nj - 1 : nj, ntask = nq * D3_ROWS;
+    const int nq = sh_dn.q != nullptr && shared ? nj - 1 : nj;
     // every pair's h into LDS by asynchronous global -> LDS copies: wavefront w copies chunks of 64 lanes, 16 bytes
     // (values) or 4 bytes (scales, sums) a lane
     const Acts a = acts_in(lds + d3_jobs_bytes(njmax), NP, ff);
@@ -390,49 +390,70 @@ __global__ void __launch_bounds__(NT, NT == 512 && is_kquant(TYPE) ? 2 : 4) k_de
         const int c = min(unit, nunit - 1), e = __builtin_amdgcn_readfirstlane(job_of(c).w);
         RowOf<TYPE, G2>::issue(v, expert_at(A, sa, e), H, row0 + row_of(c), ff, ln);
     };
-    if (threadIdx.x == 0) queue = (RING - 1) * NWV;
-#pragma unroll
-    for (int k = 0; k < RING - 1; ++k) {
-        u[k] = wv + k * NWV;
-        if (nunit > 0) request(w[k], u[k]);
-    }
-    vm_wait<0>();
-    lds_barrier();
-    // the dots, inlined once for h in LDS and once for h in global memory: a pointer that may be either is generic,
-    // and every load through it a flat load
-    auto dots = [&](const Acts& a) __attribute__((always_inline)) {
-    if (nq < nj) {
+    auto dot = [&](typename RowOf<TYPE, G2>::R& v, int unit, const Acts& a) __attribute__((always_inline)) {
+        v.prepare(ln);
+        const sfnx_job& j = job_of(unit);
+        const int n = __builtin_amdgcn_readfirstlane(j.n), r = row_of(unit);
+        for (int s = 0; s < n; ++s) {
+            const int pp = j.out[s];
+            const float d = group_sum<LPR>(v.dot(a, pp, ln));
+            if (ln == 0) part[pp][r] = d;
+        }
+    };
+    auto dense = [&](const Acts& a) __attribute__((always_inline)) {
+        if (nq == nj) return;
         const Q8sPlanes Ps = sh_dn;
         for (int task = g; task < T * D3_ROWS; task += GROUPS) {
             const int t = task / D3_ROWS, r = task % D3_ROWS;
             const float v = group_sum<LPR>(q8s_dot<LPR>(Ps, row0 + r, ff, ln, a, P + t));
             if (ln == 0) part[P + t][r] = v;
         }
-    }
-    for (bool more = true; more;) {
+    };
 #pragma unroll
-        for (int k = 0; k < RING; ++k) {
-            if (u[k] >= nunit) {   // a wavefront's units only grow: the ones after are past the last too
-                more = false;
-                break;
-            }
-            constexpr int AHEAD = RING - 1;
-            int nx = 0;
-            if (ln64 == 0) nx = atomicAdd(&queue, 1);
-            u[(k + AHEAD) % RING] = __builtin_amdgcn_readfirstlane(nx);
-            request(w[(k + AHEAD) % RING], u[(k + AHEAD) % RING]);
-            w[k].prepare(ln);
-            const sfnx_job& j = job_of(u[k]);
-            const int n = __builtin_amdgcn_readfirstlane(j.n), r = row_of(u[k]);
-            for (int s = 0; s < n; ++s) {
-                const int pp = j.out[s];
-                const float v = group_sum<LPR>(w[k].dot(a, pp, ln));
-                if (ln == 0) part[pp][r] = v;
+    for (int k = 0; k < RING - 1; ++k) u[k] = wv + k * NWV;
+    // the dots, inlined once for h in LDS and once for h in global memory: a pointer that may be either is generic,
+    // and every load through it a flat load
+    auto dots = [&](const Acts& a) __attribute__((always_inline)) {
+        if (threadIdx.x == 0) queue = (RING - 1) * NWV;
+#pragma unroll
+        for (int k = 0; k < RING - 1; ++k)
+            if (nunit > 0) request(w[k], u[k]);
+        vm_wait<0>();
+        lds_barrier();
+        dense(a);
+        for (bool more = true; more;) {
+#pragma unroll
+            for (int k = 0; k < RING; ++k) {
+                if (u[k] >= nunit) {   // a wavefront's units only grow: the ones after are past the last too
+                    more = false;
+                    break;
+                }
+                constexpr int AHEAD = RING - 1;
+                int nx = 0;
+                if (ln64 == 0) nx = atomicAdd(&queue, 1);
+                u[(k + AHEAD) % RING] = __builtin_amdgcn_readfirstlane(nx);
+                request(w[(k + AHEAD) % RING], u[(k + AHEAD) % RING]);
+                dot(w[k], u[k], a);
             }
         }
-    }
     };
-    if (staged) dots(a);
+    // Windows of few units take them all at once: no turn of the queue before a dot, and no request past the last, which were
+    // most of them.  2 rows, with the queue / without (and with the former fixed shares): Q4_K, 1024 columns, 64 experts 8.3 /
+    // 6.2 (6.6) us, 2048 columns, 512 experts 9.5 / 7.8 (8.9); Q8_0 7.3 / 6.1 (6.8) and 10.2 / 9.3 (9.9).  Not
+    // Q5_K with two groups a lane, whose second copy of the dots moves the queue's registers: 16 rows 85 -> 103 us.
+    constexpr int FEW = TYPE == SFNX_Q5_K && G2 == 2 ? 0 : RING;
+    if (FEW > 0 && staged && nunit <= FEW * NWV) {
+        typename RowOf<TYPE, G2>::R f[FEW + 1];
+#pragma unroll
+        for (int k = 0; k < FEW; ++k)
+            if (wv + k * NWV < nunit) request(f[k], wv + k * NWV);
+        vm_wait<0>();
+        lds_barrier();
+        dense(a);
+#pragma unroll
+        for (int k = 0; k < FEW; ++k)
+            if (wv + k * NWV < nunit) dot(f[k], wv + k * NWV, a);
+    } else if (staged) dots(a);
     else dots(Acts{const_cast<int8_t*>(hq_q), const_cast<float*>(hq_d), const_cast<int*>(hq_s), ff});
     __syncthreads();
     for (int i = threadIdx.x; i < T * D3_ROWS; i += NT) {

@@ -143,6 +143,31 @@ def test_fused_decode_edge_shapes(H, E, K, ff, wtype, T):
     assert max_rel(yu.cpu().numpy(), oy) < 2e-3
 
 
+@pytest.mark.parametrize("H, E, K, ff, gu, dn, q8s, T", [
+    (2560, 256, 8, 1024, orc.Q5_K, orc.Q8_0, True, 5),     # FF 1024, every down type, dense shared expert, h in LDS
+    (2560, 256, 8, 1024, orc.Q5_K, orc.Q8_0, True, 16),    # ... h in memory
+    (2560, 64, 8, 1024, orc.Q4_K, orc.Q5_1, True, 3), (1024, 64, 6, 1024, orc.Q5_1, orc.Q5_1, False, 9),
+    (1024, 64, 6, 1024, orc.Q8_0, orc.Q5_K, False, 2), (2048, 64, 6, 1024, orc.Q4_0, orc.Q5_K, True, 13),
+    (2048, 512, 10, 512, orc.Q4_0, orc.Q4_0, False, 2),    # 41 or 42 units of 48: taken at once
+    (1024, 64, 11, 512, orc.Q8_0, orc.Q8_0, False, 2),     # up to 46
+    (1024, 64, 12, 512, orc.Q8_0, orc.Q8_0, True, 2),      # up to 48
+    (1024, 64, 13, 512, orc.Q5_1, orc.Q5_1, False, 2),     # up to 54: by the queue
+    (4096, 64, 1, 512, orc.Q4_K, orc.Q4_K, False, 2), (1024, 64, 1, 512, orc.Q5_K, orc.Q4_0, True, 2)])
+def test_fused_windows_equal_unfused(H, E, K, ff, gu, dn, q8s, T):
+    """windows at FF 1024 and with few units of the down kernel: the unfused path's bits"""
+    shape = moe.LayerShape(H=H, E=E, K=K, ff=ff, wtype=gu, shared=True, dn_wtype=dn, sh_q8s=q8s)
+    L, host = make_layer(shape, 90 + T)
+    x0 = torch.from_numpy(orc.synth(T * H, 840 + T + K, 1.0).reshape(T, H)).cuda()
+    xu, xf = x0.clone(), x0.clone()
+    yu = unfused_chain([L], xu, False, [moe.DecodeBuffers(shape, T)])
+    f = moe.FusedDecode([L], T)
+    f(xf, norm=False)
+    torch.cuda.synchronize()
+    assert np.array_equal(bits(f.piece("y", torch.float32, (T, H))), bits(yu))
+    assert np.array_equal(bits(xf), bits(xu))
+    assert max_rel(yu.cpu().numpy(), orc.layer_decode(host, x0.cpu().numpy(), nthreads=8)[0]) < 2e-3
+
+
 def test_fused_decode_refuses_out_of_range():
     shape = moe.LayerShape(H=1024, E=64, K=6, ff=512, wtype=orc.Q4_K, shared=True)
     L, _ = make_layer(shape, 3)
