@@ -23,12 +23,19 @@ constexpr int MV_THREADS = 256;
 // weights from HBM: Q8_0 33.6 -> 28.9 us at 7 rows, 62 -> 50.4 at 16; Q5_1 34.6 -> 26.8, 65 -> 44.4; 1024 columns, 256
 // experts: Q8_0 99 -> 81 at 16.  Three and four tiles lost part of it again, K-quants with two took 10% more, and gate|up,
 // whose staging is a copy, gained nothing (Q8_0 71 -> 74).  Past 2048 columns two tiles' rows fill the registers.
-template <int TYPE, int G, bool DOWN> __host__ __device__ constexpr int mv_tiles() {
-    return DOWN && !is_kquant(TYPE) && G <= 4 ? 2 : 1;
+template <int TYPE, int G, bool DOWN> constexpr int mv_tiles() { return DOWN && !is_kquant(TYPE) && G <= 4 ? 2 : 1; }
+// One tile after all where the launch has little beside its longest blocks, the shared job's of T rows: those then last twice
+// as long and nothing fills the chip meanwhile.  The line is blocks (of 32 rows) a compute unit per row of the window: below
+// it 16 rows take (two tiles / one) Q8_0 31.5 / 27.3 us at 1.03 (2048 rows, top 4), 30.5 / 26.8 at 0.78, Q5_1 30.0 / 26.8 at
+// 1.03; above it 31.6 / 31.8 and 29.9 / 32.7 at 1.52, 31.6 / 38.4 and 30.4 / 39.4 at 2.0.  At 2048 columns, whose h is four
+// times as long to make, two tiles win from 1.27 (Q8_0, 16 rows 99.6 / 118.4); with 3 rows from 1.08 (Q8_0 12.0 / 13.4; at
+// 0.79 8.5 / 7.9).
+inline bool mv_two_tiles(int G, int T, int R, int njobs_max) {
+    return (long) njobs_max * ((R + 31) / 32) >= (long) (T <= 4 ? 4 : G >= 4 ? 5 : 6) * 64 * T;   // of 256 units
 }
 // TYPE: SFNX_Q4_K / SFNX_Q5_K (8 lanes a row) or SFNX_Q8_0 (16 lanes a row); G: groups or blocks per lane = C / 512;
-// TT: activation rows per pass; DOWN: activations from gu rows through swiglu (else q8_1 rows).
-template <int TYPE, int G, int TT, bool DOWN>
+// TT: activation rows per pass; DOWN: activations from gu rows through swiglu (else q8_1 rows); NTL: row tiles a block.
+template <int TYPE, int G, int TT, bool DOWN, int NTL>
 __global__ void __launch_bounds__(MV_THREADS)
 k_moe_mv(const uint8_t* __restrict__ A, size_t sa, int R, int C, const sfnx_job* __restrict__ jobs, const int* __restrict__ njobs,
          const void* __restrict__ in, float* __restrict__ out) {
@@ -42,7 +49,6 @@ k_moe_mv(const uint8_t* __restrict__ A, size_t sa, int R, int C, const sfnx_job*
     __shared__ sfnx_job jb;
     load_job(jb, jobs + ji);
     __syncthreads();
-    constexpr int NTL = mv_tiles<TYPE, G, DOWN>();
     const int r0 = blockIdx.x * NTL * RPB + threadIdx.x / LPR, ln = threadIdx.x % LPR;
     const Acts a = acts_in(lds, TT, C);
     const uint8_t* mat = expert_at(A, sa, jb.w);
@@ -67,21 +73,25 @@ k_moe_mv(const uint8_t* __restrict__ A, size_t sa, int R, int C, const sfnx_job*
 }
 
 template <int TYPE, int G, int TT, bool DOWN>
-void launch_mv(int njobs_max, size_t lds, hipStream_t s, const uint8_t* A, size_t sa, int R, int C, const sfnx_job* jobs,
+void launch_mv(int njobs_max, int T, size_t lds, hipStream_t s, const uint8_t* A, size_t sa, int R, int C, const sfnx_job* jobs,
                const int* njobs, const void* in, float* out) {
-    constexpr int rows = MV_THREADS / lpr_of<TYPE>() * mv_tiles<TYPE, G, DOWN>();
-    k_moe_mv<TYPE, G, TT, DOWN><<<dim3((R + rows - 1) / rows, njobs_max), MV_THREADS, lds, s>>>(A, sa, R, C, jobs, njobs, in, out);
+    constexpr int rows = MV_THREADS / lpr_of<TYPE>(), NTL = mv_tiles<TYPE, G, DOWN>();
+    auto go = [&](auto kern, int tiles) {
+        kern<<<dim3((R + tiles * rows - 1) / (tiles * rows), njobs_max), MV_THREADS, lds, s>>>(A, sa, R, C, jobs, njobs, in, out);
+    };
+    if (NTL > 1 && mv_two_tiles(G, T, R, njobs_max)) go(k_moe_mv<TYPE, G, TT, DOWN, NTL>, NTL);
+    else go(k_moe_mv<TYPE, G, TT, DOWN, 1>, 1);
 }
 
 template <int TYPE, int TT, bool DOWN>
-void launch_g(int G, int njobs_max, size_t lds, hipStream_t s, const uint8_t* A, size_t sa, int R, int C, const sfnx_job* jobs,
+void launch_g(int G, int njobs_max, int T, size_t lds, hipStream_t s, const uint8_t* A, size_t sa, int R, int C, const sfnx_job* jobs,
               const int* njobs, const void* in, float* out) {
     switch (G) {
-        case 1: launch_mv<TYPE, 1, TT, DOWN>(njobs_max, lds, s, A, sa, R, C, jobs, njobs, in, out); break;
-        case 2: launch_mv<TYPE, 2, TT, DOWN>(njobs_max, lds, s, A, sa, R, C, jobs, njobs, in, out); break;
-        case 4: launch_mv<TYPE, 4, TT, DOWN>(njobs_max, lds, s, A, sa, R, C, jobs, njobs, in, out); break;
-        case 5: launch_mv<TYPE, 5, TT, DOWN>(njobs_max, lds, s, A, sa, R, C, jobs, njobs, in, out); break;
-        case 8: launch_mv<TYPE, 8, TT, DOWN>(njobs_max, lds, s, A, sa, R, C, jobs, njobs, in, out); break;
+        case 1: launch_mv<TYPE, 1, TT, DOWN>(njobs_max, T, lds, s, A, sa, R, C, jobs, njobs, in, out); break;
+        case 2: launch_mv<TYPE, 2, TT, DOWN>(njobs_max, T, lds, s, A, sa, R, C, jobs, njobs, in, out); break;
+        case 4: launch_mv<TYPE, 4, TT, DOWN>(njobs_max, T, lds, s, A, sa, R, C, jobs, njobs, in, out); break;
+        case 5: launch_mv<TYPE, 5, TT, DOWN>(njobs_max, T, lds, s, A, sa, R, C, jobs, njobs, in, out); break;
+        case 8: launch_mv<TYPE, 8, TT, DOWN>(njobs_max, T, lds, s, A, sa, R, C, jobs, njobs, in, out); break;
         default: throw std::runtime_error("input width must be 512, 1024, 2048, 2560 or 4096");
     }
 }
@@ -103,7 +113,7 @@ void moe_mv(uint32_t type, const void* A, size_t sa, int n_in, int n_out, const 
     require(lds <= 64 * 1024, "activation rows do not fit the LDS budget");
     hipStream_t s = stream_of(st);
     const uint8_t* a = (const uint8_t*) A;
-#define SFNX_MV(TY, TTV) launch_g<TY, TTV, DOWN>(G, njobs_max, lds, s, a, sa, n_out, n_in, jobs, njobs, in, out)
+#define SFNX_MV(TY, TTV) launch_g<TY, TTV, DOWN>(G, njobs_max, T, lds, s, a, sa, n_out, n_in, jobs, njobs, in, out)
     if (type == SFNX_Q4_K) {
         if (TT == 1) SFNX_MV(SFNX_Q4_K, 1);
         else if (TT == 4) SFNX_MV(SFNX_Q4_K, 4);

@@ -89,3 +89,21 @@ def test_bigjobs_none(wtype):
 def test_down_few_rows(wtype, n_in, n_out):
     """the fewest rows a store holds: one or two window blocks of two row tiles"""
     test_bigjobs_equal_windows(wtype, n_in, n_out, True)
+
+
+@pytest.mark.parametrize("wtype", [orc.Q4_0, orc.Q5_1, orc.Q8_0])
+@pytest.mark.parametrize("n_in, n_out", [(512, 1040), (1024, 96), (2048, 2048)])
+def test_down_row_tiles(wtype, n_in, n_out):
+    """the window down call with one row tile a block and with two, which a larger bound on the job count selects: the
+    same bits"""
+    rng = np.random.default_rng(wtype + n_out)
+    A = store(wtype, 3, n_out, n_in, 60 + wtype)
+    _, win, P = jobs_of([1, 16, 7], rng, 20)
+    nw = torch.tensor([win.shape[0], 0], dtype=torch.int32, device="cuda")
+    x = torch.from_numpy(rng.standard_normal((20, 2 * n_in)).astype(np.float32)).cuda()
+    out = []
+    for cap in (win.shape[0], 4096):
+        out.append(torch.full((P, n_out), 7.0, device="cuda"))
+        moe.moe_down(A, n_out * moe.row_bytes(wtype, n_in), wtype, n_in, n_out, win, nw, cap, WINDOW, x, out[-1])
+    torch.cuda.synchronize()
+    assert torch.equal(out[0].view(torch.int32), out[1].view(torch.int32))
