@@ -92,7 +92,7 @@ def test_down_few_rows(wtype, n_in, n_out):
 
 
 @pytest.mark.parametrize("wtype", [orc.Q4_0, orc.Q5_1, orc.Q8_0])
-@pytest.mark.parametrize("n_in, n_out", [(512, 1040), (1024, 96), (2048, 2048)])
+@pytest.mark.parametrize("n_in, n_out", [(512, 1056), (1024, 96), (2048, 2048)])
 def test_down_row_tiles(wtype, n_in, n_out):
     """the window down call with one row tile a block and with two, which a larger bound on the job count selects: the
     same bits"""
