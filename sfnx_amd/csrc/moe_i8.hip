@@ -29,11 +29,13 @@ typedef int int4v __attribute__((ext_vector_type(4)));
 typedef int int16v __attribute__((ext_vector_type(16)));
 
 constexpr int I8_THREADS = 256, I8_WAVES = I8_THREADS / WAVE, I8_ROWS = 32 * I8_WAVES;
-// Jobs of at most i8_few rows take the decode's dot lanes (mv.hpp), a weight row's pieces all requested at once.  Only the
-// 32-value block types: their dots have no scales to unpack, and their 16 strips make the matrix-core walk longest.
-// Measured (Q8_0, 2048 columns, 512 experts, gate|up / down): 100 tokens 215 / 115 us with jobs of 1 row on the lanes, 178
-// / 127 up to 4, 166 / 146 up to 8; Q4_K 133 / 80 with none, 180 / 91 up to 4 (the walk then spills).
-constexpr int i8_few(uint32_t type, bool down) { return is_kquant(type) ? 0 : down ? 4 : 8; }
+// Jobs of at most i8_few rows take the decode's dot lanes (mv.hpp), a weight row's pieces all requested at once: the
+// matrix-core walk unpacks a step's weights for 32 tokens whatever the job holds.  Measured, the 32-value types, whose 16 strips
+// make that walk longest (Q8_0, 2048 columns, 512 experts, gate|up / down): 100 tokens 215 / 115 us with jobs of 1 row on the
+// lanes, 178 / 127 up to 4, 166 / 146 up to 8.  K-quants, gate|up from 2048 columns: jobs of 1 and 2 rows, 40 tokens, 512 experts,
+// Q4_K 84 -> 65 us, Q5_K 100 -> 82; 64 tokens, 2560 columns, 178 -> 157 and 246 -> 209; up to 4 rows lost 5% again at 100 tokens,
+// and at 1024 columns and below the walk is as short (17 tokens 15.4 -> 16.6).
+constexpr int i8_few(uint32_t type, int nr, bool down) { return is_kquant(type) ? (!down && nr >= 4 ? 2 : 0) : down ? 4 : 8; }
 constexpr float I8_M = 12582912.0f;           // 1.5 2^23
 constexpr int I8_MBITS = 0x4B400000;
 
@@ -320,14 +322,14 @@ inline int i8_grid(int nu, int njobs_cap) { return nu * ((njobs_cap + XCDS * I8_
 template <int TYPE, int NR, bool DOWN>
 __device__ __forceinline__ void few_rows(const uint8_t* mat, int R, int row0, int nrows, int n, const int* ys, const int* outs, unsigned char* lds,
                                          const void* __restrict__ in, float* __restrict__ out) {
-    constexpr int LPR = lpr_of<TYPE>(), RPB = I8_THREADS / LPR, C = 512 * NR, FEW = i8_few(TYPE, DOWN);
+    constexpr int LPR = lpr_of<TYPE>(), RPB = I8_THREADS / LPR, C = 512 * NR, FEW = i8_few(TYPE, NR, DOWN);
     const int ln = threadIdx.x % LPR, g = threadIdx.x / LPR, end = min(row0 + nrows, R);
     const Acts a = acts_in(lds, FEW, C);
     if constexpr (DOWN) stage_swiglu(a, (const float*) in, ys, n);
     else stage_q8_1(a, (const uint8_t*) in, ys, n);
     __syncthreads();
-    // two tiles' rows in registers, one requested while the other is dotted (4096 columns: one, two would spill)
-    constexpr int ND = NR < 8 ? 2 : 1;
+    // two tiles' rows in registers, one requested while the other is dotted (4096 columns, Q5_K from 2560: one, two would spill)
+    constexpr int ND = NR < (TYPE == SFNX_Q5_K ? 5 : 8) ? 2 : 1;
     typename RowOf<TYPE, NR>::R w[ND];
     if constexpr (ND == 2) RowOf<TYPE, NR>::issue(w[0], mat, R, min(row0 + g, R - 1), C, ln);
     for (int r0 = row0; r0 < end; r0 += ND * RPB)
@@ -339,6 +341,7 @@ __device__ __forceinline__ void few_rows(const uint8_t* mat, int R, int row0, in
 #pragma unroll
             for (int j = 0; j < FEW; ++j)
                 if (j < n) {
+                    if constexpr (is_kquant(TYPE)) w[p].pin();
                     const float v = group_sum<LPR>(w[p].dot(a, j, ln));
                     if (row < end && ln == 0) out[(size_t) outs[j] * R + row] = v;
                 }
@@ -366,20 +369,27 @@ __global__ void __launch_bounds__(I8_THREADS, DOWN && !is_kquant(TYPE) && NR <= 
     if (ji >= nj) return;
     ji = nj - 1 - ji;   // the shared expert's full jobs, the longest, first
     const int t0 = TOK * (u / nsl), row_base = I8_ROWS * G * (u % nsl);
-    const int n = min(TOK, jobs[ji].n - t0);
+    const int nall = jobs[ji].n;
+    // Q4_K's few rows: each token tile's block takes its share of the weight rows
+    constexpr bool SHARE = is_kquant(TYPE) && i8_few(TYPE, NR, DOWN) > 0;
+    const bool few = i8_few(TYPE, NR, DOWN) > 0 && nall <= i8_few(TYPE, NR, DOWN);
+    const int n = SHARE && few ? nall : min(TOK, nall - t0);
     if (n <= 0) return;
     __shared__ int ys[32], outs[32];
     extern __shared__ __align__(16) unsigned char lds[];
     if (threadIdx.x < 32 && (int) threadIdx.x < n) {
-        ys[threadIdx.x] = jobs[ji].y[t0 + threadIdx.x];
-        outs[threadIdx.x] = jobs[ji].out[t0 + threadIdx.x];
+        const int j0 = SHARE && few ? 0 : t0;
+        ys[threadIdx.x] = jobs[ji].y[j0 + threadIdx.x];
+        outs[threadIdx.x] = jobs[ji].out[j0 + threadIdx.x];
     }
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE, nn = lane % 32, h = lane / 32;
     const uint8_t* mat = expert_at(A, sa, jobs[ji].w);
-    if constexpr (i8_few(TYPE, DOWN) > 0)
-        if (t0 == 0 && n <= i8_few(TYPE, DOWN)) {
+    if constexpr (i8_few(TYPE, NR, DOWN) > 0)
+        if (few) {
             __syncthreads();
-            few_rows<TYPE, NR, DOWN>(mat, R, row_base, I8_ROWS * G, n, ys, outs, lds, in, out);
+            constexpr int share = SHARE ? I8_ROWS / ntt : 0;   // (G is 1 where they share)
+            if constexpr (SHARE) few_rows<TYPE, NR, DOWN>(mat, R, row_base + share * (t0 / TOK), share, n, ys, outs, lds, in, out);
+            else few_rows<TYPE, NR, DOWN>(mat, R, row_base, I8_ROWS * G, n, ys, outs, lds, in, out);
             return;
         }
     const int wrow = row_base + 32 * wave;   // the wavefront's first row
@@ -510,7 +520,7 @@ void moe_i8(uint32_t type, const void* A, size_t sa, int n_in, int n_out, const 
     int G = DOWN ? std::min(tiles, 4) : 1;
     while (G > 1 && (long) njobs_cap * ((tiles + G - 1) / G) < 1024) G /= 2;
     auto go = [&](auto kern, int tok, int strip_bytes, int lpr) {
-        const size_t lds = std::max((size_t) (DOWN ? lpr : 2) * strip_bytes, acts_bytes(i8_few(type, DOWN), n_in));
+        const size_t lds = std::max((size_t) (DOWN ? lpr : 2) * strip_bytes, acts_bytes(i8_few(type, nr, DOWN), n_in));
         if (lds > 64 * 1024) check(hipFuncSetAttribute((const void*) kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds), "hipFuncSetAttribute");
         kern<<<dim3(i8_grid((tiles + G - 1) / G * (SFNX_PF_JOB / tok), njobs_cap)), I8_THREADS, lds, stream_of(st)>>>(
             (const uint8_t*) A, sa, n_out, G, jobs, njobs, in, out);

@@ -11,7 +11,7 @@ from sfnx_amd._abi import BIGJOB_INTS, JOB_INTS, PF_JOB
 
 pytestmark = pytest.mark.gpu
 TYPES = [orc.Q4_K, orc.Q5_K, orc.Q4_0, orc.Q5_1, orc.Q8_0]
-SIZES = [1, 4, 5, 8, 9, 16, 17, 31, 32, 33, 48, 64]
+SIZES = [1, 2, 3, 4, 5, 8, 9, 16, 17, 31, 32, 33, 48, 64]
 WINDOW = 16
 
 
@@ -47,8 +47,10 @@ def jobs_of(sizes, rng, rows):
 
 @pytest.mark.parametrize("wtype", TYPES)
 @pytest.mark.parametrize("n_in, n_out", [(512, 2048), (1024, 1056), (2048, 1024), (2560, 96), (4096, 160)])
-@pytest.mark.parametrize("down", [False, True])
-def test_bigjobs_equal_windows(wtype, n_in, n_out, down):
+@pytest.mark.parametrize("down, spare", [(False, 5), (True, 5), (True, 120), (True, 400), (True, 1200)])
+def test_bigjobs_equal_windows(wtype, n_in, n_out, down, spare):
+    """spare: job slots past the jobs, which the bound on their number counts: the more, the more row tiles (1 to 4) a block of
+    down takes"""
     rng = np.random.default_rng(wtype + n_in)
     A = store(wtype, 3, n_out, n_in, 40 + wtype)
     sa = n_out * moe.row_bytes(wtype, n_in)
@@ -56,8 +58,8 @@ def test_bigjobs_equal_windows(wtype, n_in, n_out, down):
     big, win, P = jobs_of(SIZES, rng, rows)
     nb = torch.tensor([big.shape[0], 0], dtype=torch.int32, device="cuda")
     nw = torch.tensor([win.shape[0], 0], dtype=torch.int32, device="cuda")
-    cap = big.shape[0] + 5
-    big = torch.cat([big, torch.zeros((5, BIGJOB_INTS), dtype=torch.int32, device="cuda")])
+    cap = big.shape[0] + spare
+    big = torch.cat([big, torch.zeros((spare, BIGJOB_INTS), dtype=torch.int32, device="cuda")])
     x = torch.from_numpy(rng.standard_normal((rows, 2 * n_in if down else n_in)).astype(np.float32)).cuda()
     got, want = (torch.full((P, n_out), 7.0, device="cuda") for _ in range(2))
     if down:
@@ -88,7 +90,7 @@ def test_bigjobs_none(wtype):
 @pytest.mark.parametrize("n_in, n_out", [(512, 32), (1024, 64), (2048, 32)])
 def test_down_few_rows(wtype, n_in, n_out):
     """the fewest rows a store holds: one or two window blocks of two row tiles"""
-    test_bigjobs_equal_windows(wtype, n_in, n_out, True)
+    test_bigjobs_equal_windows(wtype, n_in, n_out, True, 5)
 
 
 @pytest.mark.parametrize("wtype", [orc.Q4_0, orc.Q5_1, orc.Q8_0])
