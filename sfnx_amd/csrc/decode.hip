@@ -685,9 +685,11 @@ void launch_k3(const DecArgs& d, const sfnx_moe_layer_w& w, float* x, const DecL
     // every pair's h in LDS when it fits beside the jobs and the kernel's own 11.1 KB (160 KB a workgroup on gfx950; past
     // 64 KB the kernel must be allowed the larger dynamic size first), else read from L2 per task.  148 KB holds every
     // window whose h is at most 120 KB, whatever its jobs (12 rows of 15 picks, FF 512, Q4_K: staged 21.3 us, from L2 30.7)
-    constexpr size_t DYN_MAX = 148 * 1024;
-    static_assert(acts_bytes(192, 512) == 120 * 1024 && d3_jobs_bytes(12 * 15 + 1) + acts_bytes(192, 512) <= DYN_MAX &&
-                  d3_jobs_bytes(11 * 16 + 1) + acts_bytes(11 * 17, 512) <= DYN_MAX);
+    // The 32-value types at FF 1024 read such a window's h from L2 as fast as they fetch 138 KB first, or faster (12 rows of 8 picks,
+    // 2560 columns, from L2 / staged: Q4_0 43.8 / 48.5, Q8_0 55.4 / 57.7 us; Q4_K 60.9 / 42.0, Q5_K 70.5 / 54.1), and stop at 144.
+    constexpr size_t DYN_MAX = (is_kquant(TYPE) || G2 == 1 ? 148 : 144) * 1024;
+    static_assert(acts_bytes(192, 512) == 120 * 1024);
+    static_assert(G2 != 1 || (d3_jobs_bytes(12 * 15 + 1) + acts_bytes(192, 512) <= DYN_MAX && d3_jobs_bytes(11 * 16 + 1) + acts_bytes(11 * 17, 512) <= DYN_MAX));
     // 1024 threads (4 wavefronts a SIMD: the per-pair dot chains are latency-bound) where 128 registers hold a lane's
     // tasks (FF 512; not Q5_K, whose rows carry their fifth bits)
     constexpr int NT = G2 == 1 && TYPE != SFNX_Q5_K ? 1024 : 512;
