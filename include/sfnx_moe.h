@@ -93,7 +93,7 @@ int sfnx_quantize_q8_1(const float* x, void* q, int n, int rows, void* st);
  * gates the shared expert); top-K per token among the first E by logit, ties to the lower index; weights the selected
  * softmax renormalised; jobs: one per distinct expert in first-pick order, rows in pair order (pair p = t K + k:
  * gu.y = t, gu.out = dn.y = dn.out = p).  shared != 0: one more job, expert E, rows t -> T K + t.  njobs[0] = job
- * count; njobs[1] = 0.
+ * count; njobs[1] = 0 (neither need be cleared before).
  * H % 256 == 0, H <= 4096; E % 64 == 0, E <= 1024; 1 <= K <= 16.  Pick rounds with nothing left (NaN / -inf logits)
  * write topi -1, topw 0 and leave the pair out of the jobs. */
 int sfnx_router_route(const float* W, const float* x, float* logits, int T, int H, int E, int K, int* topi, float* topw,

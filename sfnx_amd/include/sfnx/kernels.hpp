@@ -134,7 +134,7 @@ inline void router_route(const float* W, const float* x, float* logits, int T, i
                          float* sh_out = nullptr) {
     const MoeShape& s = model_shape();
     if (ec && (layer < 0 || !list)) throw std::runtime_error("router_route: a cache plan needs its layer and list");
-    // with a cache, the router launch's last block plans the window's slots, as the reference's does
+    // with a cache, the routing's launch plans the window's slots too (the reference: the router's last block)
     if (ec) ck(sfnx_router_route_plan(W, x, logits, T, s.H, s.E, s.K, topi, topw, jobs_gu, jobs_dn, njobs, 0, ec, layer, list, st));
     else ck(sfnx_router_route(W, x, logits, T, s.H, s.E, s.K, topi, topw, jobs_gu, jobs_dn, njobs, 0, st));
     if (sh_gu) ck(sfnx_q8s_gemv(sh_gu, sh_rows, s.H, sh_y, sh_out, sh_rows, T, st));

@@ -1,6 +1,6 @@
 """The expert cache (src/moe.cuh:19-71, src/kernels.cu:1636-1668): routed experts in page-locked host memory, VRAM
-slots planned per decode window by one wavefront (CLOCK), in the router launch's last block as the reference's
-(src/moe.cuh:128-198) or as a launch of its own, and filled by the copy kernel.  Each window through the cached
+slots planned per decode window by one wavefront (CLOCK), in the routing's launch (the reference: its router's last block,
+src/moe.cuh:128-198) or as a launch of its own, and filled by the copy kernel.  Each window through the cached
 layer gives the same bits as the resident layer, and the device's plan (slots, owners, refs, hand, list) equals the
 CPU restatement's (oracle/cache.py) window after window, for a pool larger and one smaller than the 32-lane sweep."""
 import numpy as np
@@ -40,7 +40,7 @@ def test_cached_decode_windows(n_slots, plan_in_router):
             moe.decode_layer_cached(cache, l, x, y1, b1, lst, plan_in_router)
             torch.cuda.synchronize()
             assert np.array_equal(bits(y0), bits(y1)), f"window {w}"
-            assert int(b1.njobs[1]) == 0   # the router's block counter left at zero
+            assert int(b1.njobs[1]) == 0   # written with the job count
             nj = int(b1.njobs[0])
             jobs = [int(v) for v in job_array(b1.jobs_gu)[:nj]["w"]]
             taken = cache_plan(st, jobs, l)

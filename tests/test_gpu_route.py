@@ -31,8 +31,8 @@ def route_case(W, x, E, K, shared):
     nj = T * K + 1
     jg = torch.full((nj * JOB_INTS,), -7, dtype=torch.int32, device="cuda")
     jd = torch.full((nj * JOB_INTS,), -7, dtype=torch.int32, device="cuda")
-    njobs = torch.zeros(2, dtype=torch.int32, device="cuda")
-    for _ in range(2):   # twice: the block counter must come back to zero
+    njobs = torch.full((2,), -7, dtype=torch.int32, device="cuda")   # both words are written, neither is read
+    for _ in range(2):
         moe.router_route(Wd, xd, logits, topi, topw, jg, jd, njobs, E, K, shared)
     torch.cuda.synchronize()
     ol = orc.router_logits(W, x)
