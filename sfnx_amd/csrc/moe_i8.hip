@@ -17,7 +17,8 @@
 //
 // Measured at 1000 tokens, 2048 columns, 512 experts x FF 512, top-10 + shared, Q4_K: gate|up 655 -> 312 us, down 620 ->
 // 239 us against one v_dot4 lane group a row (whose 16 dots a group and LDS reads this replaces); Q8_0 670 -> 390 and
-// 2,360 -> 228 us.  VALU issue takes about 70% of the SIMDs' cycles in gate|up; down adds h, made once a block.
+// 2,360 -> 228 us.  VALU issue takes 95% of the SIMDs' cycles in
+// gate|up and 80% in down (counters, 2048 tokens); down adds h, made once a block.
 #include <algorithm>
 
 #include "decode.hpp"
